@@ -74,6 +74,7 @@ class Batch {
     bool persistent_ok() const { return persistent_ok_; }
 
    private:
+    std::unique_ptr<CuShare> waiting_share(int method, int prec) const;
     struct Key {
         int bits, method, prec;
         bool operator<(const Key& o) const {

@@ -823,10 +823,18 @@ static void check_method(int method, int prec) {
     if (prec < 0 || prec > 2) throw std::invalid_argument("prec must be 0, 1 or 2");
 }
 
+// The device's CUs, where the launches of a solve may wait for each other's
+// blocks (DIC sweeps, the persistent form).
+std::unique_ptr<CuShare> Batch::waiting_share(int method, int prec) const {
+    const bool waits = prec == 2 ? sys_->dic_form() >= 2 : method == 0 && persistent_ok_;
+    return std::unique_ptr<CuShare>(waits ? new CuShare(-1) : nullptr);
+}
+
 void Batch::solve(int method, int prec, double* x, double* r1, const int* cap, const double* tol,
                   SolveResult* res, hipStream_t s) {
     check_method(method, prec);
     method = kernel_method(method);
+    const std::unique_ptr<CuShare> share = waiting_share(method, prec);
     join(s);
     const KrylovVectors<double> w = vectors64();
     std::vector<SolverState> init(k_);
@@ -887,6 +895,7 @@ void Batch::solve_mixed(int method, int prec, double* x, const double* b, double
                         hipStream_t s) {
     check_method(method, prec);
     method = kernel_method(method);
+    const std::unique_ptr<CuShare> share = waiting_share(method, prec);
     if (!(inner_rtol > 0.0 && inner_rtol < 1.0)) throw std::invalid_argument("inner_rtol must be in (0, 1)");
     join(s);
     const int n = n_tot_, T = tile0_[k_];

@@ -27,7 +27,7 @@
 #include <initializer_list>
 #include <type_traits>
 
-#include "krylov_kernels.h"
+#include "cg_resident.h"
 
 namespace tflows {
 
@@ -57,7 +57,6 @@ __device__ __forceinline__ bool block_halted(const SolverState* st) {
 // kReplaceDrop times the FP64 norm of the last replacement (so the FP32
 // recurrence never runs far past the accuracy FP32 can attain).  Returns
 // true when iteration kd must not run.
-constexpr double kReplaceDrop = 1e-2;
 
 // The state fields a kernel's stopping test and scalars read, loaded
 // together at its start: the test then waits for one memory round trip

@@ -1,0 +1,977 @@
+// cg_resident.hip -- Jacobi (or unpreconditioned) CG with the vectors of the
+// solve kept on the chip: one launch runs many iterations, one block per CU.
+//
+// What bounds the kernel-per-phase form (cg_fused.hip) is not arithmetic:
+// every iteration moves x, r, z, p, q and D through memory (10 N values
+// beside the SpMV) and pays three kernel starts.  The register files and the
+// LDS of 256 CUs hold 168 MB, so here x, r, D, z / q and the matrix rows of a
+// block stay in registers and p in LDS for the whole launch.
+//
+// k_cg_window, the form of the meshes: a block also keeps p of the rows of
+// other blocks that its columns reach (its halo), and advances it itself:
+// p = z + beta p needs only their z, which is published before the
+// reduction that gives beta.  Per iteration:
+//
+//   C  ||r||^2 and rho = (r, z) over all blocks, z published
+//                                      -> stopping test, beta, own and halo p
+//   B  (p, q) over all blocks          -> alfa
+//
+// so an iteration costs two synchronisations, one write of z, one read of
+// the halo's z, and gathers from LDS.
+//
+// k_cg_stream: any matrix (rows of any length, columns anywhere): the rows
+// are read every iteration and p is published, which takes a third
+// synchronisation (A: a block waits for the blocks its columns reach).  It
+// sums over the same rows in the same order, so both give the same bits.
+//
+// Process/CG.f90:113-259 per iteration, every value formed with the
+// reference's operations in the reference's order (each row's products added
+// in CSR order); only the dot-product summation order is the blocks'.
+//
+// Synchronisation without fences: values that cross blocks (z or p, and the
+// partial sums) are stored and loaded with device-coherent accesses that
+// bypass the non-coherent caches, so no L2 is written back or invalidated.
+// A block posts its partial sums in words that carry the number of the
+// synchronisation beside 32 bits of the value; a reader polls all blocks'
+// words until every one carries that number, and adds the values in block
+// order: every block gets the same bits.  B and C alternate and each waits
+// for every block, so one set of words per site is enough: no block can post
+// its next B before all have read the last C, and none posts C before all
+// have read the last B.
+//
+// Every wait ends: the grid is at most one block per CU (the host checks
+// that the device holds it at once), and a wait longer than wait_ticks
+// (another process held the CUs) raises the fault word, on which every
+// block stops; the host then restores the vectors and runs the
+// kernel-per-phase form.
+#include <algorithm>
+#include <condition_variable>
+#include <cstdlib>
+#include <mutex>
+#include <type_traits>
+
+#include "cg_resident.h"
+
+namespace tflows {
+
+namespace {
+
+constexpr int kResWaves = kResThreads / kWave;
+// one block up to this many rows: its synchronisations are block barriers
+constexpr int kResOneBlockRows = 4096;
+// else blocks of at least this many: below it the synchronisation of more
+// blocks costs more than the shorter row sums save; up to twice as many
+// where that keeps to the blocks that synchronise in one step (84,480 rows,
+// locality order: 64 blocks 11.6 ms, 80 blocks 13.9)
+constexpr int kResMinRows = 1024;
+
+__device__ __forceinline__ double coherent_load(const double* p) {
+    const uint64_t u = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(double, u);
+}
+__device__ __forceinline__ float coherent_load(const float* p) {
+    const uint32_t u = __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(float, u);
+}
+__device__ __forceinline__ void coherent_store(double* p, double v) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void coherent_store(float* p, float v) {
+    __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Posts of one site: word i of block b at i * stride + b, so that a
+// wavefront polls 64 blocks' words in four cache lines, and where every
+// block reads them in kPostCopies copies, one for the blocks of each XCD
+// (one copy: 7500 cycles against 3700 at 32 blocks).  Each word carries 32
+// bits of the value and the tag.
+template <typename T> struct PostWords;
+template <> struct PostWords<double> { static constexpr int n = 2; };
+template <> struct PostWords<float> { static constexpr int n = 1; };
+
+__device__ __forceinline__ void post_word(uint64_t* w, uint32_t v, uint32_t tag) {
+    __hip_atomic_store(w, ((uint64_t)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void post_value(uint64_t* w, int stride, double v, uint32_t tag) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    post_word(w, (uint32_t)b, tag);
+    post_word(w + stride, (uint32_t)(b >> 32), tag);
+}
+[[maybe_unused]] __device__ __forceinline__ void post_value(uint64_t* w, int, float v, uint32_t tag) {
+    post_word(w, __builtin_bit_cast(uint32_t, v), tag);
+}
+// true (and v) when every word of the value carries the tag
+__device__ __forceinline__ bool read_value(const uint64_t* w, int stride, uint32_t tag, double& v) {
+    const uint64_t a = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t b = __hip_atomic_load(w + stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = __builtin_bit_cast(double, (a & 0xffffffffu) | (b << 32));
+    return (uint32_t)(a >> 32) == tag && (uint32_t)(b >> 32) == tag;
+}
+__device__ __forceinline__ bool read_value(const uint64_t* w, int, uint32_t tag, float& v) {
+    const uint64_t a = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = __builtin_bit_cast(float, (uint32_t)a);
+    return (uint32_t)(a >> 32) == tag;
+}
+
+// Waits of one launch: bounded by the wall clock and the fault word.
+struct Waiter {
+    int* fault;
+    uint64_t ticks;
+    HostMirror* hm;                 // told, too, so that a host that paces itself on it stops
+    // false when the wait must be given up
+    __device__ __forceinline__ bool keep_waiting(unsigned& polls, uint64_t& t0) const {
+        if ((++polls & 127u) != 0) return true;
+        const uint64_t now = (uint64_t)wall_clock64();
+        if (polls == 128u) t0 = now;
+        if (now - t0 > ticks || __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+            __hip_atomic_store(fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            publish(hm, 1, 0);
+            return false;
+        }
+        return true;
+    }
+};
+
+// Sum over the block of value k of every thread, in wavefront k's lanes.  The
+// values go through LDS and one wavefront adds them: a cross-lane sum in
+// every wavefront cost 4 x 40 instructions on each SIMD.
+template <typename T, int NV>
+__device__ __forceinline__ T block_partial(int tid, const T (&v)[NV], T* sm) {
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) sm[k * kResThreads + tid] = v[k];
+    __syncthreads();
+    T s = T(0);
+    if (w < NV) {
+        T t[kResWaves];
+#pragma unroll
+        for (int i = 0; i < kResWaves; ++i) t[i] = sm[w * kResThreads + i * kWave + lane];
+        s = t[0];
+#pragma unroll
+        for (int i = 1; i < kResWaves; ++i) s += t[i];
+        s = wave_sum(s);
+    }
+    return s;
+}
+
+// Sums of NV values over the block, valid in every thread.
+template <typename T, int NV>
+__device__ __forceinline__ void block_total(T (&v)[NV], T* sm) {
+    __shared__ T tot[NV];
+    const T s = block_partial<T, NV>(threadIdx.x, v, sm);
+    if (threadIdx.x % kWave == 0 && threadIdx.x / kWave < NV) tot[threadIdx.x / kWave] = s;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = tot[k];
+}
+
+// Polls the posts of value k of blocks b0 + lane * step (lane < count) and
+// returns their sum in every lane of the wavefront.
+template <typename T>
+__device__ __forceinline__ T poll_sum(const uint64_t* slots, int k, int stride, int b, bool use, uint32_t tag,
+                                      const Waiter& wt, int* s_fail) {
+    T got = T(0);
+    if (use) {
+        const uint64_t* s = slots + k * PostWords<T>::n * stride + b;
+        unsigned polls = 0;
+        uint64_t t0 = 0;
+        while (!read_value(s, stride, tag, got))
+            if (!wt.keep_waiting(polls, t0)) {
+                *s_fail = 1;
+                break;
+            }
+    }
+    return wave_sum(got);
+}
+
+// Sums of NV values over the block, then over the `nblk` blocks (posted in
+// `slots`).  Valid in every thread; false when the wait was given up (the
+// whole block agrees).  Up to a wavefront of blocks each reads all posts;
+// above that the first block of each eighth adds its eighth's posts and posts
+// the sum, and every block reads eight: all blocks reading all posts took
+// 9000 cycles at 256 blocks, two steps take 6200 (one at 32 blocks: 3300).
+template <typename T, int NV>
+__device__ __forceinline__ bool resident_sum(int tid, T (&v)[NV], uint64_t* slots, int nblk, int blk, uint32_t tag,
+                                             const Waiter& wt, int* s_fail, T* sm) {
+    __shared__ T tot[NV];
+    constexpr int kWords = PostWords<T>::n;
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+    T s = block_partial<T, NV>(tid, v, sm);
+    if (w < NV && nblk > 1) {
+        const bool flat = nblk <= kWave;
+        const int m = nblk / kNumXcd, g = flat ? 0 : blk / m;        // above kWave blocks, a multiple of 8
+        bool poster = true;
+        if (!flat) {
+            if (lane == 0) post_value(slots + w * kWords * kPostStride + blk, kPostStride, s, tag);
+            poster = blk == g * m;
+            if (poster) s = poll_sum<T>(slots, w, kPostStride, blk + lane, lane < m, tag, wt, s_fail);
+            slots += kPostCopies * kPostSite;
+        }
+        const int stride = flat ? kPostStride : kNumXcd, copy = flat ? kPostSite : kPostSecond;
+        if (poster && lane < kPostCopies)
+            post_value(slots + lane * copy + w * kWords * stride + (flat ? blk : g), stride, s, tag);
+        s = poll_sum<T>(slots + (blockIdx.x & (kPostCopies - 1)) * copy, w, stride, lane, lane < (flat ? nblk : kNumXcd),
+                        tag, wt, s_fail);
+    }
+    if (w < NV && lane == 0) tot[w] = s;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = tot[k];
+    return *s_fail == 0;
+}
+
+// A vector of other blocks' values, read W (16 bytes of) rows at a time with
+// device-coherent loads (the same cache policy as the atomic loads above: a
+// wider access needs no atomicity, since the rows of a granule are complete
+// before the synchronisation that precedes the load).
+template <typename T>
+struct CoherentVec {
+    static constexpr int W = 16 / (int)sizeof(T);
+    static constexpr int kSc1 = 16;                  // device scope, in the builtin's policy bits
+    __amdgpu_buffer_rsrc_t rsrc;
+    const T* v;
+    int n;
+    __device__ __forceinline__ CoherentVec(const T* vec, int n_)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(vec), 0, n_ * (int)sizeof(T), 0x00027000)), v(vec),
+          n(n_) {}
+    // rows c .. c + W - 1, which lie in the vector
+    __device__ __forceinline__ void load(int c, T (&out)[W]) const {
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c * (int)sizeof(T), 0, kSc1);
+        __builtin_memcpy(out, &q, sizeof(out));
+    }
+};
+
+// `count` granules of consecutive rows from `row` on, at lp[at] (16-byte
+// aligned).
+struct HaloRun {
+    int at, row, count;
+};
+
+// The first NB granules of a run that a thread moves: loaded, then applied
+// as p = z + beta p.  A run that reaches outside the matrix (the first and
+// last blocks') is left to apply, row by row.
+template <typename T, int NB>
+struct HaloLoad {
+    static constexpr int W = CoherentVec<T>::W;
+    T z[NB][W];
+    __device__ __forceinline__ static bool inside(const CoherentVec<T>& v, const HaloRun& h) {
+        return h.row >= 0 && h.row + h.count * W <= v.n;
+    }
+    __device__ __forceinline__ void load(int tid, const CoherentVec<T>& v, const HaloRun& h, int e0 = 0) {
+        if (!inside(v, h)) return;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int e = e0 + i * kResThreads + tid;
+            if (e < h.count) v.load(h.row + e * W, z[i]);
+        }
+    }
+    __device__ __forceinline__ void apply(int tid, const CoherentVec<T>& v, T* lp, const HaloRun& h, bool first, T beta,
+                                          int e0 = 0) {
+        if (inside(v, h)) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int e = e0 + i * kResThreads + tid;
+                if (e < h.count)
+#pragma unroll
+                    for (int u = 0; u < W; ++u)
+                        lp[h.at + e * W + u] = first ? z[i][u] : z[i][u] + beta * lp[h.at + e * W + u];
+            }
+            return;
+        }
+        for (int e = e0 * W + tid; e < min(h.count, e0 + NB * kResThreads) * W; e += kResThreads) {
+            const int c = h.row + e;
+            if (c < 0 || c >= v.n) continue;
+            const T zc = coherent_load(v.v + c);
+            lp[h.at + e] = first ? zc : zc + beta * lp[h.at + e];
+        }
+    }
+    __device__ __forceinline__ void rest(int tid, const CoherentVec<T>& v, T* lp, const HaloRun& h, bool first, T beta) {
+        for (int e0 = NB * kResThreads; e0 < h.count; e0 += NB * kResThreads) {
+            load(tid, v, h, e0);
+            apply(tid, v, lp, h, first, beta, e0);
+        }
+    }
+};
+
+// p of a column: this block's rows in LDS, others from memory with
+// device-coherent loads (a row the entry lacks reads LDS slot 0: unused).
+template <typename T>
+struct ResGather {
+    const T* lp;
+    const T* __restrict__ pg;
+    int rb, nloc;
+    __device__ __forceinline__ T operator()(bool has, int c) const {
+        const unsigned o = (unsigned)(c - rb);
+        const bool loc = o < (unsigned)nloc;
+        T g = lp[loc ? o : 0];
+        // a 32-bit byte offset from a scalar base (n * sizeof(T) < 2^32)
+        if (has && !loc)
+            g = coherent_load(reinterpret_cast<const T*>(reinterpret_cast<const char*>(pg) +
+                                                         (uint32_t)c * (uint32_t)sizeof(T)));
+        return g;
+    }
+};
+
+// The slots of a row kept in registers: values and where the column's p is
+// in LDS, in CSR order.  A slot the row lacks has the value 0 and a finite p
+// (its own row, or the place of a row outside the matrix, which holds 0), so
+// it adds +-0 to a sum that is never -0: the sum's bits are those of the
+// slots it has.
+template <typename Op> struct OpDiff { static constexpr bool value = false; };
+template <> struct OpDiff<DiffSell32> { static constexpr bool value = true; };
+template <typename T, bool SHARED>
+struct RowSlots {
+    static constexpr int N = window_slots<T>();
+    T a[N];
+    int c[SHARED ? 1 : N];
+    T rs;                           // difference form: the row sum
+};
+
+// Row `row` (every thread of the block calls it, with live = false past the
+// block's rows: the slice is the wavefront's, clamped to the last one).
+// Shared offsets: slot j is the matrix's j-th column offset, whose p lies
+// w.disp[j] from the row's own in LDS, so no index is kept.  Otherwise c is
+// an index of lp (own: the row's).
+template <bool SHARED, typename Op, typename T>
+__device__ __forceinline__ void load_row(const Op& A, int row, bool live, const WindowShape& w, int base, int own,
+                                         RowSlots<T, SHARED>& s) {
+    constexpr int N = RowSlots<T, SHARED>::N;
+    const int lane = (int)threadIdx.x & (kSlice - 1);
+    const int sl = __builtin_amdgcn_readfirstlane(min(row, A.n - 1) / kSlice);
+    row = sl * kSlice + lane;
+    const int b = A.off[sl];
+    const int stored = (A.off[sl + 1] - b) / kSlice;
+    if constexpr (OpDiff<Op>::value) s.rs = live ? A.rs[row] : T(0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) s.a[j] = T(0);
+    if constexpr (SHARED) {
+        const bool sym = A.lbase != nullptr;
+        const int sb = sym ? A.sidx[sl] : b / kSlice;
+        const int ws = sym ? A.sidx[sl + 1] - sb : stored;
+        const int nl = ws - stored;
+        const unsigned m = live ? A.mask[row] : 0u;
+        for (int i = 0; i < ws; ++i) {               // the slice's slots; both lists ascend
+            const int d = __builtin_amdgcn_readfirstlane(A.soff[sb + i]);
+            if (!((m >> i) & 1u)) continue;
+            const T v = A.val[i < nl ? sym_mirror_pos(A.lbase, sb, i, sl, row, d) : b + lane + (i - nl) * kSlice];
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+                if (j < w.nslots && d == w.offset[j]) s.a[j] = v;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            s.c[j] = own;
+            if (!live || j >= stored) continue;
+            const int at = b + lane + j * kSlice;
+            int c = -1;
+            if (A.dc) {
+                const short d = A.dc[at];
+                if (d != kPad16) c = row + (int)d;
+            } else {
+                c = A.col[at];
+            }
+            if (c >= 0) {
+                s.c[j] = c - base;
+                s.a[j] = A.val[at];
+            }
+        }
+    }
+}
+
+// Products added to 0 in CSR order (CG.f90:193-199), or the terms of the
+// difference form, gathered from LDS; `off` is an opaque 0.  Row k of a thread lies k * kResThreads above its first, an
+// immediate offset of the LDS reads.
+template <bool SHARED, typename Op, typename T>
+__device__ __forceinline__ T row_sum(const RowSlots<T, SHARED>& s, int k, int own, int off, const WindowShape& w,
+                                     const T* lp) {
+    constexpr int N = RowSlots<T, SHARED>::N;
+    T acc = T(0);
+    T pv[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        if constexpr (SHARED) pv[j] = (lp + own + w.disp[j])[k * kResThreads];
+        else pv[j] = lp[off + s.c[j]];
+    }
+    const T pi = OpDiff<Op>::value ? (lp + own)[k * kResThreads] : T(0);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        acc = acc + s.a[j] * (OpDiff<Op>::value ? pv[j] - pi : pv[j]);
+    if constexpr (OpDiff<Op>::value) acc = acc + s.rs * pi;
+    return acc;
+}
+
+// Rows of any width, read from memory slot by slot.
+template <typename T>
+__device__ __forceinline__ T stream_row(const Sell<T>& A, int row, const ResGather<T>& g) {
+    const int sl = __builtin_amdgcn_readfirstlane(row / kSlice);
+    const int b = A.off[sl] + row - sl * kSlice;
+    const int w = (A.off[sl + 1] - A.off[sl]) / kSlice;
+    T acc = T(0);
+#pragma unroll 4
+    for (int j = 0; j < w; ++j) {
+        int c = -1;
+        if (A.dc) {
+            const short d = A.dc[b + j * kSlice];
+            if (d != kPad16) c = row + (int)d;
+        } else {
+            c = A.col[b + j * kSlice];
+        }
+        const T sum = acc + A.val[b + j * kSlice] * g(c >= 0, c);
+        acc = c >= 0 ? sum : acc;
+    }
+    return acc;
+}
+template <typename T>
+__device__ __forceinline__ T stream_row(const Csr<T>& A, int row, const ResGather<T>& g) {
+    T acc = T(0);
+    const int e1 = A.rowptr[row + 1];
+#pragma unroll 4
+    for (int e = A.rowptr[row]; e < e1; ++e) acc = acc + A.val[e] * g(true, A.col[e]);
+    return acc;
+}
+
+}  // namespace
+
+template <typename Op, int R, typename T = typename OpValue<Op>::type>
+__global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T> a) {
+    extern __shared__ __align__(16) char res_lds[];
+    T* lp = reinterpret_cast<T*>(res_lds);           // p of this block's rows
+    __shared__ T sm[2 * kResThreads];
+    __shared__ int s_fail, s_done;
+    SolverState* st = a.st;
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        s_fail = 0;
+        s_done = st->done;
+    }
+    const int G = gridDim.x, blk = logical_block();
+    const int rb = min(blk * a.rows, a.n), nloc = min(a.n - rb, a.rows);
+    const bool lead = blk == 0 && tid == 0;
+    const double tol = st->tol;
+    const int cap = st->cap, it0 = st->it;
+    T rho_old = (T)st->rho[it0 & 1];
+    __syncthreads();
+    if (s_done) return;
+    const Waiter wt{&st->fault, a.wait_ticks, a.hm};
+    const ResGather<T> g{lp, a.p, rb, nloc};
+    const int alo = G > 1 ? a.deps[2 * blk] / a.rows : 0, ahi = G > 1 ? a.deps[2 * blk + 1] / a.rows : 0;
+    T xv[R], rv[R], dv[R], zq[R];   // zq: z, then q of the iteration
+#pragma unroll
+    for (int k = 0; k < R; ++k) {   // past the block's rows: x = r = p = 0, D = 1, no entries
+        const int l = k * kResThreads + tid;
+        T d = T(1), p = T(0);
+        xv[k] = rv[k] = zq[k] = T(0);
+        if (l < nloc) {
+            xv[k] = a.x[rb + l];
+            rv[k] = a.r[rb + l];
+            d = a.D[rb + l];
+            if (it0 > 0) p = a.p[rb + l];
+            if (a.keep) {           // the state a fallback starts from
+                a.keep[rb + l] = xv[k];
+                a.keep[(size_t)a.n + rb + l] = rv[k];
+            }
+        }
+        lp[l] = p;
+        dv[k] = d;
+    }
+    uint32_t tag = a.tag;
+    int it = it0, niter = 0;
+    bool stop = false;
+    double err = 0.0;
+    for (;;) {
+        T v[2] = {T(0), T(0)};
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            zq[k] = rv[k] / dv[k];                       // z, CG.f90:126
+            v[0] += rv[k] * rv[k];                       // ||r||^2, CG.f90:250
+            v[1] += rv[k] * zq[k];                       // rho, CG.f90:174
+        }
+        if (!resident_sum<T, 2>(tid, v, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
+        err = sqrt((double)v[0]);
+        if (err < tol) {                                 // CG.f90:93-108, :248-255
+            stop = true;
+            niter = it;
+            break;
+        }
+        if (it + 1 > cap) {                              // CG.f90:259-262
+            stop = true;
+            niter = (cap > 0 ? cap : 0) + 1;
+            break;
+        }
+        if (it - it0 == a.chunk) break;
+        const T rho = v[1];
+        const bool first = it == 0;
+        const T beta = first ? T(0) : rho / rho_old;     // CG.f90:183
+        rho_old = rho;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + tid;
+            const T p = first ? zq[k] : zq[k] + beta * lp[l];       // CG.f90:180, :185
+            lp[l] = p;
+            if (G > 1 && l < nloc) coherent_store(a.p + rb + l, p);
+        }
+        if (G > 1) {
+            ++tag;
+            __builtin_amdgcn_s_waitcnt(0);               // this wave's p stores have reached memory
+            __syncthreads();
+            if (tid == 0) __hip_atomic_store(a.flags + blk, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int b = alo + tid;
+            if (b <= ahi && b != blk) {
+                unsigned polls = 0;
+                uint64_t t0 = 0;
+                while ((int)(__hip_atomic_load(a.flags + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - tag) < 0)
+                    if (!wt.keep_waiting(polls, t0)) {
+                        s_fail = 1;
+                        break;
+                    }
+            }
+        }
+        __syncthreads();
+        if (s_fail) return;
+        T pq[1] = {T(0)};
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + tid;
+            zq[k] = l < nloc ? stream_row(A, rb + l, g) : T(0);     // CG.f90:193-199
+            pq[0] += lp[l] * zq[k];                                 // CG.f90:216
+        }
+        if (!resident_sum<T, 1>(tid, pq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
+        const T alfa = rho / pq[0];                      // CG.f90:219
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + tid;
+            xv[k] = xv[k] + alfa * lp[l];                // CG.f90:227
+            rv[k] = rv[k] - alfa * zq[k];                // CG.f90:228
+        }
+        ++it;
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int l = k * kResThreads + tid;
+        if (l < nloc) {
+            a.x[rb + l] = xv[k];
+            a.r[rb + l] = rv[k];
+            if (G == 1) a.p[rb + l] = lp[l];
+        }
+    }
+    if (lead) {
+        st->it = it;
+        st->rho[it & 1] = (double)rho_old;
+        st->error = err;
+        if (stop) {
+            st->done = 1;
+            st->niter_out = niter;
+        }
+    }
+}
+
+// SHARED: shared-offset matrix, the halo being `lo` rows either side and the
+// far regions of w; else the halo is the window of columns the block reaches
+// (deps).  LDS: halo below, own rows, halo above, far regions.
+template <typename Op, bool SHARED, int R, bool MIXED, typename T = typename OpValue<Op>::type>
+__global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T> a, WindowShape w) {
+    extern __shared__ __align__(16) char res_lds[];
+    __shared__ T sm[2 * kResThreads];
+    __shared__ int s_fail, s_done;
+    SolverState* st = a.st;
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        s_fail = 0;
+        s_done = st->done | st->suspend | st->fault;
+    }
+    const int G = gridDim.x, blk = logical_block();
+    const int rb = min(blk * a.rows, a.n), nloc = min(a.n - rb, a.rows);
+    const bool lead = blk == 0 && tid == 0;
+    const double tol = st->tol;
+    const int cap = st->cap, it0 = st->it;
+    double err_rep = st->err_rep;
+    T rho_old = (T)st->rho[it0 & 1];
+    __syncthreads();
+    if (s_done) return;
+    const Waiter wt{&st->fault, a.wait_ticks, a.hm};
+    int lo = w.lo, hi = w.lo;
+    if (!SHARED) {                  // the columns this block reaches
+        lo = G > 1 && nloc > 0 ? halo_rows(rb - a.deps[2 * blk]) : 0;
+        hi = G > 1 && nloc > 0 ? halo_rows(a.deps[2 * blk + 1] + 1 - (rb + a.rows)) : 0;
+    }
+    constexpr bool kLdsD = window_d_in_lds<T>(R);
+    T* const ld = reinterpret_cast<T*>(res_lds);     // D where it is in LDS, else nothing
+    T* const lp = ld + (kLdsD ? R * kResThreads : 0);
+    T* const own = lp + lo;
+    for (size_t i = tid; i < w.lds / sizeof(T); i += kResThreads) ld[i] = T(0);   // read as a finite p (times 0) too
+    __syncthreads();
+    T xv[R], rv[R], dv[kLdsD ? 1 : R], zq[R];        // zq: z, then q of the iteration
+    RowSlots<T, SHARED> rows[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {   // past the block's rows: x = r = 0, D = 1, no entries
+        const int l = k * kResThreads + tid;
+        T d = T(1);
+        xv[k] = rv[k] = zq[k] = T(0);
+        if (l < nloc) {
+            xv[k] = a.x[rb + l];
+            rv[k] = a.r[rb + l];
+            d = a.D[rb + l];
+            if (a.keep) {           // the state a fallback starts from
+                a.keep[rb + l] = xv[k];
+                a.keep[(size_t)a.n + rb + l] = rv[k];
+            }
+        }
+        if (it0 > 0 && l < nloc) own[l] = a.p[rb + l];
+        if (kLdsD) ld[l] = d;
+        else dv[kLdsD ? 0 : k] = d;
+        load_row(A, rb + l, l < nloc, w, rb - lo, lo + min(l, a.rows - 1), rows[k]);
+    }
+    // The halo: runs of rows in LDS order, moved W rows (16 bytes) at a time.
+    // A run's rows may lie partly outside the matrix.
+    constexpr int W = 16 / (int)sizeof(T);
+    const CoherentVec<T> zin(a.z, a.n);
+    const HaloRun below{0, rb - lo, lo / W}, above{lo + a.rows, rb + a.rows, hi / W};
+    auto far = [&](int q) { return HaloRun{w.farbase + q * a.rows, rb + w.far[q], q < w.nfar ? a.rows / W : 0}; };
+    auto first_p = [&](const HaloRun& h) {
+        for (int e = tid; it0 > 0 && e < h.count * W; e += kResThreads)
+            if (h.row + e >= 0 && h.row + e < a.n) lp[h.at + e] = a.p[h.row + e];
+    };
+    first_p(below);
+    first_p(above);
+    if (SHARED)
+        for (int q = 0; q < w.nfar; ++q) first_p(far(q));
+    double err64 = 0.0;
+    if (MIXED) {                    // the FP64 norm of the replacement before this launch (site E)
+        __shared__ double sm64[kResThreads];
+        double e[1] = {0.0};
+        for (int b = tid; b < a.nE; b += kResThreads) e[0] += a.partE[b];
+        block_total<double, 1>(e, sm64);
+        err64 = sqrt(e[0]);
+    }
+    uint32_t tag = a.tag;
+    int it = it0, niter = 0;
+    bool stop = false, pause = false;
+    double err = 0.0;
+    for (;;) {
+        // opaque, as the same every iteration the compiler would keep all
+        // addresses formed from it in registers
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        T v[2] = {T(0), T(0)};
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + t;
+            zq[k] = rv[k] / (kLdsD ? ld[l] : dv[kLdsD ? 0 : k]);    // z, CG.f90:126
+            v[0] += rv[k] * rv[k];                                  // ||r||^2, CG.f90:250
+            v[1] += rv[k] * zq[k];                                  // rho, CG.f90:174
+            if (G > 1 && l < nloc) coherent_store(a.z + rb + l, zq[k]);
+        }
+        __builtin_amdgcn_s_waitcnt(0);               // this wave's z has reached memory before the block posts
+        if (!resident_sum<T, 2>(t, v, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
+        err = sqrt((double)v[0]);
+        if (MIXED && it == it0) {                    // after a replacement the FP64 norm decides
+            err = err_rep = err64;
+            if (lead) {
+                st->error = st->err_rep = err;
+                if (it == 0) {
+                    st->ini_res = err;
+                    st->ini_written = 1;
+                }
+            }
+        } else if (MIXED) {
+            pause = err < kReplaceDrop * err_rep || err < tol;      // the next replacement verifies
+            if (pause) break;
+        }
+        if (err < tol) {                             // CG.f90:93-108, :248-255
+            stop = true;
+            niter = it;
+            break;
+        }
+        if (it + 1 > cap) {                          // CG.f90:259-262
+            stop = true;
+            niter = (cap > 0 ? cap : 0) + 1;
+            break;
+        }
+        if (it - it0 == a.chunk) break;
+        const T rho = v[1];
+        const bool first = it == 0;
+        const T beta = first ? T(0) : rho / rho_old;                // CG.f90:183
+        rho_old = rho;
+        if (G > 1) {                                 // the halo's p, every run's loads in flight together
+            constexpr int NF = (R + W - 1) / W;      // granules of a far run per thread
+            if constexpr (SHARED) {
+                HaloLoad<T, NF> f0, f1;
+                HaloLoad<T, 1> n0, n1;
+                f0.load(t, zin, far(0));
+                f1.load(t, zin, far(1));
+                n0.load(t, zin, below);
+                n1.load(t, zin, above);
+                f0.apply(t, zin, lp, far(0), first, beta);
+                f1.apply(t, zin, lp, far(1), first, beta);
+                n0.apply(t, zin, lp, below, first, beta);
+                n1.apply(t, zin, lp, above, first, beta);
+                n0.rest(t, zin, lp, below, first, beta);
+                n1.rest(t, zin, lp, above, first, beta);
+                if (w.nfar > 2) {
+                    f0.load(t, zin, far(2));
+                    f1.load(t, zin, far(3));
+                    f0.apply(t, zin, lp, far(2), first, beta);
+                    f1.apply(t, zin, lp, far(3), first, beta);
+                }
+            } else {
+                HaloLoad<T, 4> n0, n1;
+                n0.load(t, zin, below);
+                n1.load(t, zin, above);
+                n0.apply(t, zin, lp, below, first, beta);
+                n1.apply(t, zin, lp, above, first, beta);
+                n0.rest(t, zin, lp, below, first, beta);
+                n1.rest(t, zin, lp, above, first, beta);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + t;
+            if (l < nloc) own[l] = first ? zq[k] : zq[k] + beta * own[l];
+        }
+        __syncthreads();
+        T pq[1] = {T(0)};
+        int at = lo + t, off = 0;
+        asm volatile("" : "+v"(off));
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + t;
+            zq[k] = row_sum<SHARED, Op>(rows[k], k, at, off, w, lp);
+            if (l < nloc) pq[0] += own[l] * zq[k];                  // CG.f90:216
+            if (R > 2) asm volatile("" : "+v"(zq[k]));              // one row's gathers in registers at a time
+        }
+        if (!resident_sum<T, 1>(t, pq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
+        const T alfa = rho / pq[0];                                 // CG.f90:219
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kResThreads + t;
+            if (l < nloc) xv[k] = xv[k] + alfa * own[l];            // CG.f90:227
+            rv[k] = rv[k] - alfa * zq[k];                           // CG.f90:228
+        }
+        ++it;
+        if (MIXED && it - it0 == a.chunk) break;
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int l = k * kResThreads + tid;
+        if (l < nloc) {
+            a.x[rb + l] = xv[k];
+            a.r[rb + l] = rv[k];
+            a.p[rb + l] = own[l];
+        }
+    }
+    if (lead) {
+        st->it = it;
+        st->rho[it & 1] = (double)rho_old;
+        if (!MIXED) st->error = err;
+        if (pause) st->suspend = 1;
+        if (stop) {
+            st->done = 1;
+            st->niter_out = niter;
+            publish(a.hm, 1, it);
+        }
+    }
+}
+
+// Smallest and largest column of each block's rows.
+__global__ __launch_bounds__(kBlock) void k_resident_deps(int n, int rows, const int* __restrict__ rowptr,
+                                                          const int* __restrict__ col, int* __restrict__ deps) {
+    __shared__ int lo, hi;
+    if (threadIdx.x == 0) {
+        lo = n;
+        hi = 0;
+    }
+    __syncthreads();
+    const int b = blockIdx.x;
+    const int rb = min(b * rows, n), re = min(n, rb + rows);
+    int l = n, h = 0;
+    if (rb < re)
+        for (int e = rowptr[rb] + (int)threadIdx.x; e < rowptr[re]; e += kBlock) {
+            l = min(l, col[e]);
+            h = max(h, col[e]);
+        }
+    atomicMin(&lo, l);
+    atomicMax(&hi, h);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        deps[2 * b] = rb < re ? lo : min(b * rows, n - 1);
+        deps[2 * b + 1] = rb < re ? hi : min(b * rows, n - 1);
+    }
+}
+
+bool cg_resident_enabled() {
+    const char* e = std::getenv("TFLOWS_CG_RESIDENT");
+    return !(e && e[0] == '0') && !std::getenv("TFLOWS_CG_FORM") && !std::getenv("TFLOWS_CG_CARRY");
+}
+
+static int device_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    return cus;
+}
+
+uint64_t resident_wait_ticks() {
+    const char* e = std::getenv("TFLOWS_BARRIER_WAIT_MS");
+    const long ms = e ? std::atol(e) : 2000;
+    int dev = 0, khz = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
+        khz = 100000;
+    return (uint64_t)khz * (uint64_t)(ms < 0 ? 0 : ms);
+}
+
+ResidentShape resident_shape(int n, int rows_per_thread) {
+    ResidentShape r;
+    const int cus = std::min(device_cus(), kResMaxBlocks);
+    if (n <= 0 || cus <= 0) return r;
+    int grid = 1;
+    if (n > kResOneBlockRows) {
+        grid = std::min(cus, (n + kResMinRows - 1) / kResMinRows);
+        if (grid > kWave && n <= kWave * 2 * kResMinRows) grid = kWave;
+        if (grid >= kNumXcd) grid = grid / kNumXcd * kNumXcd;   // whole shares of the XCDs
+    }
+    const int64_t rows = (((int64_t)n + grid - 1) / grid + kSlice - 1) / kSlice * kSlice;
+    if (rows > (int64_t)rows_per_thread * kResThreads) return r;
+    r.grid = grid;
+    r.rows = (int)rows;
+    return r;
+}
+
+namespace {
+struct CuPool {
+    std::mutex m;
+    std::condition_variable cv;
+    uint64_t next = 0, serving = 0;
+    int used = 0, cap = 0;
+};
+CuPool g_cu_pools[64];
+}  // namespace
+
+CuShare::CuShare(int blocks) : dev_(0), blocks_(blocks) {
+    if (hipGetDevice(&dev_) != hipSuccess || dev_ < 0 || dev_ >= 64) dev_ = 0;
+    CuPool& p = g_cu_pools[dev_];
+    std::unique_lock<std::mutex> lk(p.m);
+    if (p.cap == 0) p.cap = std::max(1, device_cus());
+    if (blocks_ < 0 || blocks_ > p.cap) blocks_ = p.cap;
+    const uint64_t mine = p.next++;
+    p.cv.wait(lk, [&] { return p.serving == mine && p.used + blocks_ <= p.cap; });
+    p.used += blocks_;
+    ++p.serving;
+    p.cv.notify_all();
+}
+CuShare::~CuShare() {
+    CuPool& p = g_cu_pools[dev_];
+    std::lock_guard<std::mutex> lk(p.m);
+    p.used -= blocks_;
+    p.cv.notify_all();
+}
+
+void launch_resident_deps(int n, int rows, int grid, const int* rowptr, const int* col, int* deps, hipStream_t s) {
+    hipLaunchKernelGGL(k_resident_deps, dim3(grid), dim3(kBlock), 0, s, n, rows, rowptr, col, deps);
+}
+
+// Launches `kernel` on `grid` blocks if the device holds them all at once.
+template <class K, class... Args>
+static bool launch_resident(K kernel, int grid, size_t lds, hipStream_t s, const Args&... args) {
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kernel, kResThreads, lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (per_cu <= 0 || grid > per_cu * cus) return false;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kResThreads), lds, s, args...);
+    return true;
+}
+
+// values of LDS: own rows and halo (the reads of the threads past the
+// block's rows stay inside), and D
+template <typename T>
+static size_t window_elems(const ResidentShape& sh, int lo, int hi, int nfar) {
+    const int R = window_kernel_rows((sh.rows + kResThreads - 1) / kResThreads);
+    return (size_t)lo + hi + (size_t)nfar * sh.rows + (size_t)R * kResThreads * (window_d_in_lds<T>(R) ? 2 : 1);
+}
+
+template <typename T>
+bool window_shape(const ResidentShape& sh, const std::vector<int>& offsets, WindowShape& w) {
+    w = WindowShape{};
+    if ((int)offsets.size() > window_slots<T>()) return false;
+    for (int d : offsets) {
+        const int64_t ad = d < 0 ? -(int64_t)d : d;
+        if (ad < sh.rows) w.lo = std::max(w.lo, halo_rows((int)ad));
+        else if (w.nfar < kMaxFar) w.far[w.nfar++] = d;
+        else return false;
+    }
+    w.farbase = 2 * w.lo + sh.rows;
+    for (int d : offsets) {
+        w.disp[w.nslots] = d;
+        for (int f = 0; f < w.nfar; ++f)
+            if (w.far[f] == d) w.disp[w.nslots] = w.farbase + f * sh.rows - w.lo;
+        w.offset[w.nslots++] = d;
+    }
+    w.lds = sizeof(T) * window_elems<T>(sh, w.lo, w.lo, w.nfar);
+    return w.lds <= kResLdsBytes;
+}
+template <typename T>
+bool window_shape(const ResidentShape& sh, const std::vector<int>& deps, int n, WindowShape& w) {
+    w = WindowShape{};
+    size_t most = window_elems<T>(sh, 0, 0, 0);
+    for (int b = 0; b < sh.grid && sh.grid > 1 && (int64_t)b * sh.rows < n; ++b)
+        most = std::max(most, window_elems<T>(sh, halo_rows(b * sh.rows - deps[2 * b]),
+                                              halo_rows(deps[2 * b + 1] + 1 - (b + 1) * sh.rows), 0));
+    w.lds = sizeof(T) * most;
+    return w.lds <= kResLdsBytes;
+}
+template bool window_shape<double>(const ResidentShape&, const std::vector<int>&, WindowShape&);
+template bool window_shape<float>(const ResidentShape&, const std::vector<int>&, WindowShape&);
+template bool window_shape<double>(const ResidentShape&, const std::vector<int>&, int, WindowShape&);
+template bool window_shape<float>(const ResidentShape&, const std::vector<int>&, int, WindowShape&);
+
+template <typename Op, typename T>
+bool launch_cg_stream(const Op& A, const ResidentArgs<T>& a, int grid, hipStream_t s) {
+    const int R = (a.rows + kResThreads - 1) / kResThreads;
+    const size_t lds = sizeof(T) * (size_t)((R + 1) / 2 * 2) * kResThreads;
+    if (R <= 2) return launch_resident(k_cg_stream<Op, 2>, grid, lds, s, A, a);
+    if (R <= 4) return launch_resident(k_cg_stream<Op, 4>, grid, lds, s, A, a);
+    if (R <= 6) return launch_resident(k_cg_stream<Op, 6>, grid, lds, s, A, a);
+    return launch_resident(k_cg_stream<Op, 8>, grid, lds, s, A, a);
+}
+template bool launch_cg_stream<Sell<double>, double>(const Sell<double>&, const ResidentArgs<double>&, int,
+                                                     hipStream_t);
+template bool launch_cg_stream<Csr<double>, double>(const Csr<double>&, const ResidentArgs<double>&, int, hipStream_t);
+
+// the kernel of the fewest rows per thread that hold R (even ones, the FP32
+// ones above 8 by fours)
+template <bool SHARED, int N, typename Op, typename T>
+static bool launch_window(std::integral_constant<int, N>, int R, const Op& A, const ResidentArgs<T>& a,
+                          const WindowShape& w, int grid, hipStream_t s) {
+    if constexpr (N > resident_rows_per_thread<T>(!SHARED)) {
+        return false;
+    } else {
+        if (R <= N) return launch_resident(k_cg_window<Op, SHARED, N, OpDiff<Op>::value>, grid, w.lds, s, A, a, w);
+        return launch_window<SHARED>(std::integral_constant<int, window_kernel_rows(N + 1)>{}, R, A, a, w,
+                                     grid, s);
+    }
+}
+
+template <typename Op, typename T>
+bool launch_cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, int grid, hipStream_t s) {
+    const int R = (a.rows + kResThreads - 1) / kResThreads;
+    return A.soff ? launch_window<true>(std::integral_constant<int, 1>{}, R, A, a, w, grid, s)
+                  : launch_window<false>(std::integral_constant<int, 1>{}, R, A, a, w, grid, s);
+}
+template bool launch_cg_window<Sell<double>, double>(const Sell<double>&, const ResidentArgs<double>&,
+                                                     const WindowShape&, int, hipStream_t);
+template bool launch_cg_window<DiffSell32, float>(const DiffSell32&, const ResidentArgs<float>&, const WindowShape&,
+                                                  int, hipStream_t);
+
+}  // namespace tflows

@@ -56,6 +56,7 @@ struct SolverState {
     // replacement does not apply it again.
     double alfa;
     int xupd;
+    int fault;                      // raised by a wait of the on-chip CG that was given up
 };
 
 // Host-visible mirror of the end of a solve, written by the device with

@@ -256,6 +256,7 @@ DiffSell32 System::sell32(hipStream_t s) {
             TF_CHECK(hipMemcpy(sell_mask_.p, mask.data(), mask.size(), hipMemcpyHostToDevice));
             sell_col_.release();
             sell_dc_.release();
+            slot_summary(off, soff, sell_offsets_, sell_width_);
             // the symmetric form where the pattern allows it; the values are
             // checked at every change (below)
             SymSlots sym;
@@ -279,6 +280,7 @@ DiffSell32 System::sell32(hipStream_t s) {
             sell_soff_.release();
             sell_mask_.release();
             slice_layout(n_, orp, ocol, true, off, col, map);
+            slot_summary(off, {}, sell_offsets_, sell_width_);
             sell_col_.ensure(col.size());
             if (!col.empty())
                 TF_CHECK(hipMemcpy(sell_col_.p, col.data(), sizeof(int) * col.size(), hipMemcpyHostToDevice));
@@ -633,7 +635,41 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
     mirror32_->iter = 0;
     // the FP64 residual on the operator of the FP64 iterations (sliced or
     // CSR: the same bits)
-    const bool carry = cg_form() != 2 && cg_carry();
+    // The FP32 iterations between two replacements on the chip where they
+    // fit: one launch of cg_resident.hip each
+    const ResidentShape shape =
+        cg_resident_enabled() && interval <= 4 * kResChunk ? resident_shape_of<float>() : ResidentShape{};
+    ResidentSpace sp;
+    WindowShape win;
+    bool resident = false;
+    if (shape.grid) {
+        sp = resident_space(shape, true, s);
+        resident = window_of(shape, sell32(s), sell_width_, sell_offsets_, win);
+    }
+    const DiffSell32 A32 = resident ? sell32(s) : DiffSell32{};
+    std::unique_ptr<CuShare> share;
+    if (resident) {
+        share.reset(new CuShare(shape.grid));
+        TF_CHECK(hipMemcpyAsync(sp.keep, x, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+    }
+    ResidentArgs<float> ra{};
+    ra.n = n_;
+    ra.rows = shape.rows;
+    ra.chunk = interval;
+    ra.x = x32;
+    ra.r = r32;
+    ra.p = p0;
+    ra.z = z;
+    ra.D = D32;
+    ra.slotB = sp.posts;
+    ra.slotC = sp.posts + kPostTotal / 2;
+    ra.deps = sp.deps;
+    ra.partE = partE;
+    ra.nE = grid_;
+    ra.wait_ticks = resident_wait_ticks();
+    ra.st = state32_.p;
+    ra.hm = mirror32_;
+    const bool carry = !resident && cg_form() != 2 && cg_carry();
     auto replace = [&](double* rout) {
         if (carry)
             hipLaunchKernelGGL(k_rel_merge_carry, dim3(nb), dim3(kBlock), 0, s, n_, x, x32, (const float*)p0,
@@ -669,7 +705,12 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
         }
     };
     while (!done && issued <= guard) {
-        with_op32(s, iterations);
+        if (resident) {
+            ra.tag = *sp.tag;
+            *sp.tag += resident_tags(interval);
+            resident = launch_cg_window(A32, ra, win, shape.grid, s);
+        }
+        if (!resident) with_op32(s, iterations);
         issued += interval;
         replace(nullptr);
         ++replacements;
@@ -693,6 +734,12 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
     const double fin = std::sqrt(host_site_sum(partE, grid_, s));
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
+    if (h2.fault) {      // a launch gave up waiting: from the initial x again, one launch per kernel
+        share.reset();
+        resident_gave_up();
+        TF_CHECK(hipMemcpyAsync(x, sp.keep, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+        return solve_mixed_reliable_impl(prec, x, b, r_out, cap, tol, interval, outer_steps, s);
+    }
     SolveResult res;
     res.ini_res = h2.ini_res;
     res.ini_written = h2.ini_written != 0;

@@ -4,11 +4,11 @@
 // system) lives in one file-scope device array, `scratch`, of fixed size.
 //
 // The kernels are the ones System::solve runs for CG with Jacobi or no
-// preconditioning (the three-kernel iteration: stopping test and p update,
-// SpMV with (p, q), x / r update), on the system's CSR arrays; the sliced
-// operator System::solve may pick gives the same row sums bit for bit, and
-// both sum the dot products over the same tiles, so the results are the
-// same bits.  BiCG runs through the CG kernels, as System::solve does: the
+// preconditioning (the on-chip form of cg_resident.hip, else the
+// three-kernel iteration: stopping test and p update, SpMV with (p, q),
+// x / r update), on the system's CSR arrays; the sliced operator
+// System::solve may pick gives the same row sums bit for bit, and both sum
+// the dot products over the same rows, so the results are the same bits.  BiCG runs through the CG kernels, as System::solve does: the
 // reference's shadow system reproduces the primal one (BiCG.f90:93-95,
 // 196-200).
 //
@@ -34,7 +34,9 @@ constexpr int kNoAllocMaxGrid = 4096;
 constexpr size_t kStateDoubles = 64;                              // 512 B, one SolverState
 constexpr size_t kPartialDoubles = 8 * (size_t)kNoAllocMaxGrid;   // Sites<double>::elems(grid)
 constexpr size_t kVectorDoubles = 6 * (size_t)kNoAllocMaxRows;    // D, p, q, z, x and r1 in internal order
-constexpr size_t kScratchDoubles = kStateDoubles + kPartialDoubles + kVectorDoubles;
+// on-chip CG: posts of two sites, a flag and the block reach of every block
+constexpr size_t kPostDoubles = (size_t)kPostTotal + 2 * (size_t)kResMaxBlocks;
+constexpr size_t kScratchDoubles = kStateDoubles + kPartialDoubles + kPostDoubles + kVectorDoubles;
 static_assert(sizeof(SolverState) <= kStateDoubles * sizeof(double), "SolverState outgrew its scratch slot");
 
 static __device__ __align__(256) double scratch[kScratchDoubles];
@@ -104,7 +106,8 @@ SolveResult solve_noalloc(System& S, int method, int prec, double* x, double* r1
     double* base = device_scratch();
     SolverState* st = reinterpret_cast<SolverState*>(base);
     double* partials = base + kStateDoubles;
-    double* vec = partials + kPartialDoubles;
+    double* posts = partials + kPartialDoubles;
+    double* vec = posts + kPostDoubles;
     const size_t nn = (size_t)n;
     KrylovVectors<double> w;
     w.D = vec;
@@ -120,6 +123,7 @@ SolveResult solve_noalloc(System& S, int method, int prec, double* x, double* r1
     }
     const unsigned zb = (unsigned)std::min<size_t>(2048, (4 * nn + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(k_zero, dim3(zb), dim3(kBlock), 0, s, 4 * nn, vec);
+    hipLaunchKernelGGL(k_zero, dim3(64), dim3(kBlock), 0, s, kPostDoubles, posts);
     hipLaunchKernelGGL(k_state_init, dim3(1), dim3(kWave), 0, s, st, tol, cap, stale_error);
     TF_CHECK(hipGetLastError());
     if (reord) {
@@ -132,11 +136,33 @@ SolveResult solve_noalloc(System& S, int method, int prec, double* x, double* r1
     static const Levels kNoLevels;
     start_solve<double, Csr<double>>(c, 0, prec, A, A, w, sites, st, nullptr, &kNoLevels, s, false, false);
     TF_CHECK(hipGetLastError());
+    // on the chip, as System::solve does, where it fits
+    SolverState h;
+    bool resident = false;
+    const ResidentShape shape = cg_resident_enabled() ? S.resident_shape_of<double>() : ResidentShape{};
+    if (shape.grid) {
+        SolverState h0{};
+        h0.tol = tol;
+        h0.cap = cap;
+        h0.error = stale_error;
+        launch_cgf_check(false, sites, (const double*)nullptr, st, nullptr, s);
+        uint32_t tag = 0;
+        System::ResidentSpace sp;
+        sp.posts = reinterpret_cast<uint64_t*>(posts);
+        sp.flags = reinterpret_cast<uint32_t*>(posts + (size_t)kPostTotal);
+        sp.deps = reinterpret_cast<int*>(posts + (size_t)kPostTotal + kResMaxBlocks);
+        sp.keep = w.q;                  // q and z, which the on-chip form does not use
+        sp.tag = &tag;
+        sp.deps_ready = false;
+        auto launch = [&](const ResidentArgs<double>& a) { return launch_cg_stream(A, a, shape.grid, s); };
+        resident = S.run_resident(shape, sp, launch, w, st, h0, h, s);
+        if (!resident) launch_cgf_init_z(n, (const double*)w.r1, (const double*)w.D, w.u1, sites, st, s);
+    }
     // Iterations in chunks (4, doubling to 64); after each chunk the host
     // waits for the stream and reads the device's `done` flag.  Kernels
     // queued past convergence return at once.
     int issued = 0, chunk = 4;
-    bool done = false;
+    bool done = resident;
     while (issued < cap && !done) {
         const int k = std::min(chunk, cap - issued);
         for (int i = 0; i < k; ++i) {
@@ -152,11 +178,12 @@ SolveResult solve_noalloc(System& S, int method, int prec, double* x, double* r1
     }
     if (!done) launch_check(c, std::max(cap, 0) + 1, sites, st, nullptr, s);
     // the x update of the last iteration, which no p kernel applied
-    if (carries_x(c, 0, true)) launch_cg_xfinish(A.n, w.x, (const double*)w.p, st, s);
+    if (!resident && carries_x(c, 0, true)) launch_cg_xfinish(A.n, w.x, (const double*)w.p, st, s);
     TF_CHECK(hipGetLastError());
-    SolverState h;
-    TF_CHECK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
-    TF_CHECK(hipStreamSynchronize(s));
+    if (!resident) {
+        TF_CHECK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
+        TF_CHECK(hipStreamSynchronize(s));
+    }
     if (!h.done) throw HipError("solver finished without reaching a stopping state");
     if (reord) {
         S.to_external((const double*)w.x, x, s);

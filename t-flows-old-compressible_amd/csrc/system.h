@@ -3,11 +3,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <memory>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
+#include "cg_resident.h"
 #include "krylov_kernels.h"
 #include "slot_layout.h"
 
@@ -137,6 +139,8 @@ bool slot_offsets16(int n, const std::vector<int>& off, const std::vector<int>& 
 bool col16_from_env(const char* name);
 void slice_layout(int n, const std::vector<int>& rp, const std::vector<int>& cl, bool pad_own, std::vector<int>& off,
                   std::vector<int>& col, std::vector<int>& map);
+// the distinct column offsets and the most slots of a slice of a sliced layout
+void slot_summary(const std::vector<int>& off, const std::vector<int>& soff, std::vector<int>& offsets, int& width);
 bool shared_slots_from_env();
 
 // Whether the FP64 (TFLOWS_SYM_SLOTS, default on) or the FP32
@@ -360,6 +364,7 @@ class System {
     template <class F>
     SolveResult dic_retry(double* const* vecs, int count, hipStream_t s, F&& f) {
         if (dic_form() < 2) return f();
+        const CuShare share(-1);   // its sweeps' wavefronts wait for each other, too
         dic_backup_.ensure((size_t)count * n_);
         for (int k = 0; k < count; ++k)
             TF_CHECK(hipMemcpyAsync(dic_backup_.p + (size_t)k * n_, vecs[k], sizeof(double) * n_,
@@ -377,7 +382,37 @@ class System {
     template <typename T>
     void dic_apply(const Csr<T>& A, const T* D, const T* u, T* z, const SolverState* st, hipStream_t s);
 
+    // Buffers of the on-chip CG (cg_resident.hip), from the system's own
+    // memory or a caller's.
+    struct ResidentSpace {
+        uint64_t* posts = nullptr;   // sites B and C: 2 x kPostStride words per block
+        uint32_t* flags = nullptr;   // one per block
+        int* deps = nullptr;         // 2 per block (filled when a run starts)
+        double* keep = nullptr;      // 2 n: what a fallback starts from
+        uint32_t* tag = nullptr;     // host: number of the last synchronisation
+        bool deps_ready = true;      // deps holds the blocks' columns already
+    };
+    // The iterations of a started Jacobi CG solve on the chip, to their end
+    // (h: the state read back); launch(args) starts one launch.  False when a
+    // wait was given up or the device does not hold the grid: x, r1 and the
+    // state are as before the first iteration again.
+    bool run_resident(const ResidentShape& shape, const ResidentSpace& sp,
+                      const std::function<bool(const ResidentArgs<double>&)>& launch, const KrylovVectors<double>& w,
+                      SolverState* st, const SolverState& h0, SolverState& h, hipStream_t s);
+    // blocks and rows of the on-chip CG (grid 0: not this system)
+    template <typename T>
+    ResidentShape resident_shape_of() const {
+        return res_off_ ? ResidentShape{} : resident_shape(n_, resident_rows_per_thread<T>(reordered_));
+    }
+
    private:
+    void resident_gave_up();
+    ResidentSpace resident_space(const ResidentShape& shape, bool keep, hipStream_t s);
+    // halo of k_cg_window for a sliced operator; false: the rows are too
+    // long or the LDS too small
+    template <typename Op>
+    bool window_of(const ResidentShape& shape, const Op& A, int width, const std::vector<int>& offsets,
+                   WindowShape& w) const;
     SolveResult solve_ext(int method, int prec, double* x, double* r1, int cap, double tol, double stale_error,
                           hipStream_t s);
     SolveResult solve_impl(int method, int prec, double* x, double* r1, int cap, double tol, double stale_error,
@@ -435,6 +470,16 @@ class System {
     bool sym64_refused_ = false, sym32_refused_ = false;   // values seen that are not symmetric
     DevArray<int> symflag_;
     int op64_mode_ = 2;
+    int op64_env_ = 2;              // the choice of the environment (2: none)
+    DevArray<uint64_t> res_posts_;  // on-chip CG: posts, flags, block reach, fallback copies
+    DevArray<uint32_t> res_flags_;
+    DevArray<int> res_deps_;
+    DevArray<double> res_keep_;
+    uint32_t res_tag_ = 0;
+    std::vector<int> res_deps_h_;
+    std::vector<int> sell64_offsets_, sell_offsets_;   // distinct column offsets of the shared-offset layouts
+    int sell64_width_ = 0, sell_width_ = 0;            // most slots of a slice
+    bool res_off_ = false;          // a wait was given up: kernel per phase from now on
     DevArray<float> off_val_, rowsum32_, diag32_;
     bool diff32_valid_ = false;
     DevArray<int> tpos_;
@@ -447,6 +492,7 @@ class System {
     Levels levels_;
     bool levels_ready_ = false;
     DevArray<double> dic_backup_;   // inputs of a DIC solve, for dic_retry
+    int max_row_ = 0;               // most entries of a row
     int grid_;
     int lanes_ = 1;
     int strided_ = 0;

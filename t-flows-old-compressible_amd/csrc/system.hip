@@ -153,6 +153,14 @@ void slice_layout(int n, const std::vector<int>& rp, const std::vector<int>& cl,
     }
 }
 
+void slot_summary(const std::vector<int>& off, const std::vector<int>& soff, std::vector<int>& offsets, int& width) {
+    offsets = soff;
+    std::sort(offsets.begin(), offsets.end());
+    offsets.erase(std::unique(offsets.begin(), offsets.end()), offsets.end());
+    width = 0;
+    for (size_t sl = 0; sl + 1 < off.size(); ++sl) width = std::max(width, (off[sl + 1] - off[sl]) / kSlice);
+}
+
 bool shared_slots_from_env() {
     const char* e = std::getenv("TFLOWS_SHARED_SLOTS");
     return !(e && e[0] == '0');
@@ -230,6 +238,7 @@ Sell<double> System::sell64(hipStream_t s) {
             TF_CHECK(hipMemcpy(sell64_mask_.p, mask.data(), mask.size(), hipMemcpyHostToDevice));
             sell64_col_.release();
             sell64_dc_.release();
+            slot_summary(off, soff, sell64_offsets_, sell64_width_);
             // the symmetric form where the pattern allows it; the values are
             // checked at every change (below)
             SymSlots sym;
@@ -253,6 +262,7 @@ Sell<double> System::sell64(hipStream_t s) {
             sell64_soff_.release();
             sell64_mask_.release();
             slice_layout(n_, rp, cl, false, off, col, map);
+            slot_summary(off, {}, sell64_offsets_, sell64_width_);
             sell64_col_.ensure(col.size());
             TF_CHECK(hipMemcpy(sell64_col_.p, col.data(), sizeof(int) * col.size(), hipMemcpyHostToDevice));
             // 16-bit column offsets where every one fits (TFLOWS_FP64_COL16=0
@@ -338,7 +348,7 @@ System::System(int n, int nonz, const int* acol, const int* arow, const int* adi
                hipStream_t s, bool allow_reorder)
     : n_(n), nnz_(nonz - 1), grid_(stream_grid(n, max_blocks_from_env())), lanes_(lanes_from_env()),
       strided_(tile_order_from_env()), op32_mode_(op_mode_from_env("TFLOWS_FP32_OP")),
-      op64_mode_(op_mode_from_env("TFLOWS_FP64_OP")) {
+      op64_mode_(op_mode_from_env("TFLOWS_FP64_OP")), op64_env_(op64_mode_) {
     if (n <= 0) throw std::invalid_argument("N must be positive");
     if (nonz < n + 1) throw std::invalid_argument("NONZ must be at least N + 1 (diagonal entries + 1)");
     rowptr_.ensure(n_ + 1);
@@ -366,6 +376,7 @@ System::System(int n, int nonz, const int* acol, const int* arow, const int* adi
         if (h_dia_[i] < h_rowptr_[i] || h_dia_[i] >= h_rowptr_[i + 1])
             throw std::invalid_argument("Adia(i) must point inside row i");
     }
+    for (int i = 0; i < n_; ++i) max_row_ = std::max(max_row_, h_rowptr_[i + 1] - h_rowptr_[i]);
     for (int i = 0; i < n_ + 1; ++i) h_rowptr_[i] -= 1;
     for (int i = 0; i < n_; ++i) h_dia_[i] -= 1;
     for (int j = 0; j < nnz_; ++j) {
@@ -784,6 +795,8 @@ void System::prec1(int prec, double* d_ext, hipStream_t s) {
     TF_CHECK(hipMemsetAsync(ws_.p, 0, sizeof(double) * n_, s));
     double* d = reordered_ ? ext_buffer(0) : d_ext;
     if (prec == 2) {
+        std::unique_ptr<CuShare> share;
+        if (dic_form() >= 2) share.reset(new CuShare(-1));
         dic_setup(d, s);
         if (dic_form() >= 2) {
             try {
@@ -1133,6 +1146,95 @@ SolveResult System::solve_ext(int method, int prec, double* x, double* r1, int c
     return res;
 }
 
+void System::resident_gave_up() {
+    res_off_ = true;
+    std::fprintf(stderr, "libtflows_krylov: an on-chip CG launch gave up waiting (TFLOWS_BARRIER_WAIT_MS); this "
+                         "system now runs one launch per kernel\n");
+    std::fflush(stderr);
+}
+
+System::ResidentSpace System::resident_space(const ResidentShape& shape, bool keep, hipStream_t s) {
+    const size_t words = kPostTotal;
+    if (!res_posts_.p || res_tag_ > (1u << 30)) {   // the synchronisations are numbered from 1 over zeroed words
+        res_posts_.ensure(words);
+        res_flags_.ensure(shape.grid);
+        TF_CHECK(hipMemsetAsync(res_posts_.p, 0, sizeof(uint64_t) * words, s));
+        TF_CHECK(hipMemsetAsync(res_flags_.p, 0, sizeof(uint32_t) * shape.grid, s));
+        res_tag_ = 0;
+    }
+    if (keep) res_keep_.ensure(2 * (size_t)n_);
+    if (!res_deps_.p && shape.grid > 1) {           // the pattern, and so the shape, is the system's for good
+        res_deps_.ensure(2 * (size_t)shape.grid);
+        res_deps_h_.resize(2 * (size_t)shape.grid);
+        launch_resident_deps(n_, shape.rows, shape.grid, rowptr_.p, col_.p, res_deps_.p, s);
+        TF_CHECK(hipGetLastError());
+        TF_CHECK(hipMemcpyAsync(res_deps_h_.data(), res_deps_.p, sizeof(int) * res_deps_h_.size(),
+                                hipMemcpyDeviceToHost, s));
+        TF_CHECK(hipStreamSynchronize(s));
+    }
+    ResidentSpace sp;
+    sp.posts = res_posts_.p;
+    sp.flags = res_flags_.p;
+    sp.deps = res_deps_.p;
+    sp.keep = res_keep_.p;
+    sp.tag = &res_tag_;
+    return sp;
+}
+
+bool System::run_resident(const ResidentShape& shape, const ResidentSpace& sp,
+                          const std::function<bool(const ResidentArgs<double>&)>& launch,
+                          const KrylovVectors<double>& w, SolverState* st, const SolverState& h0, SolverState& h,
+                          hipStream_t s) {
+    const CuShare share(shape.grid);
+    if (!sp.deps_ready && shape.grid > 1)
+        launch_resident_deps(n_, shape.rows, shape.grid, rowptr_.p, col_.p, sp.deps, s);
+    ResidentArgs<double> a{};
+    a.n = n_;
+    a.rows = shape.rows;
+    a.chunk = kResChunk;
+    a.x = w.x;
+    a.r = w.r1;
+    a.p = w.p;
+    a.z = w.u1;
+    a.D = w.D;
+    a.slotB = sp.posts;
+    a.slotC = sp.posts + kPostTotal / 2;
+    a.flags = sp.flags;
+    a.deps = sp.deps;
+    a.wait_ticks = resident_wait_ticks();
+    a.st = st;
+    a.keep = sp.keep;
+    for (;;) {
+        a.tag = *sp.tag;
+        *sp.tag += resident_tags(a.chunk);
+        if (!launch(a)) return false;
+        TF_CHECK(hipGetLastError());
+        TF_CHECK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
+        TF_CHECK(hipStreamSynchronize(s));
+        if (h.fault) break;
+        if (h.done) return true;
+        a.keep = nullptr;
+    }
+    TF_CHECK(hipMemcpyAsync(w.x, sp.keep, sizeof(double) * n_, hipMemcpyDeviceToDevice, s));
+    TF_CHECK(hipMemcpyAsync(w.r1, sp.keep + n_, sizeof(double) * n_, hipMemcpyDeviceToDevice, s));
+    TF_CHECK(hipMemcpyAsync(st, &h0, sizeof(h0), hipMemcpyHostToDevice, s));
+    TF_CHECK(hipStreamSynchronize(s));
+    return false;
+}
+
+template <typename Op>
+bool System::window_of(const ResidentShape& shape, const Op& A, int width, const std::vector<int>& offsets,
+                       WindowShape& w) const {
+    using T = typename OpValue<Op>::type;
+    if (width > window_slots<T>()) return false;
+    if (!A.soff && shape.rows > resident_rows_per_thread<T>(true) * kResThreads) return false;
+    return A.soff ? window_shape<T>(shape, offsets, w) : window_shape<T>(shape, res_deps_h_, n_, w);
+}
+template bool System::window_of<Sell<double>>(const ResidentShape&, const Sell<double>&, int, const std::vector<int>&,
+                                              WindowShape&) const;
+template bool System::window_of<DiffSell32>(const ResidentShape&, const DiffSell32&, int, const std::vector<int>&,
+                                            WindowShape&) const;
+
 int kernel_method(int method) {
     if (method != 1) return method;
     const char* e = std::getenv("TFLOWS_BICG_SHADOW");
@@ -1145,9 +1247,13 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     method = kernel_method(method);
     ws_.ensure((size_t)V_COUNT * n_);
     KrylovVectors<double> w = vectors(x, r1);
+    // CG on the chip where it fits (it reads no workspace that it or its
+    // set-up has not written)
+    const ResidentShape shape =
+        method == 0 && prec != 2 && cg_resident_enabled() ? resident_shape_of<double>() : ResidentShape{};
     // iteration 1 overwrites p, p2, u1, u2 before reading them; zero the
     // workspace anyway so no value of a previous solve lingers
-    TF_CHECK(hipMemsetAsync(ws_.p, 0, sizeof(double) * (size_t)V_COUNT * n_, s));
+    if (!shape.grid) TF_CHECK(hipMemsetAsync(ws_.p, 0, sizeof(double) * (size_t)V_COUNT * n_, s));
 
     SolverState h{};
     h.tol = tol;
@@ -1161,12 +1267,38 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     const Levels* L = prec == 2 ? &levels() : &kNoLevels;
     if (prec == 2) prepare_dic(false, s);
     const Csr<double> A = csr();
-    with_op64(s, [&](const auto& Aop) {
-        run_solve<double, std::decay_t<decltype(Aop)>>(ctx(), method, prec, cap, Aop, A, w, sites(), state_.p,
-                                                       mirror_, L, s, false, false, &replay_);
-    });
     SolverState h2;
-    TF_CHECK(hipMemcpy(&h2, state_.p, sizeof(h2), hipMemcpyDeviceToHost));
+    bool resident = false;
+    if (shape.grid) {
+        start_solve<double, Csr<double>>(ctx(), method, prec, A, A, w, sites(), state_.p, mirror_, L, s, false, false);
+        launch_cgf_check(false, sites(), (const double*)nullptr, state_.p, mirror_, s);   // CG.f90:93-108
+        const ResidentSpace sp = resident_space(shape, true, s);
+        // the sliced operator, unless TFLOWS_FP64_OP=csr or rows of very
+        // uneven length pad it far
+        const bool csr_rows = op64_env_ == 0 || (sell64(s), sell64_entries_ > nnz_ + nnz_ / 2 + 64 * (int64_t)kSlice);
+        WindowShape win;
+        const bool window = !csr_rows && window_of(shape, sell64(s), sell64_width_, sell64_offsets_, win);
+        auto launch = [&](const ResidentArgs<double>& a) {
+            if (window) return launch_cg_window(sell64(s), a, win, shape.grid, s);
+            return csr_rows ? launch_cg_stream(A, a, shape.grid, s) : launch_cg_stream(sell64(s), a, shape.grid, s);
+        };
+        resident = run_resident(shape, sp, launch, w, state_.p, h, h2, s);
+        if (!resident) {
+            resident_gave_up();
+            launch_cgf_init_z(n_, (const double*)w.r1, (const double*)w.D, w.u1, sites(), state_.p, s);
+        }
+    }
+    if (!resident) {
+        with_op64(s, [&](const auto& Aop) {
+            if (shape.grid)
+                pace_iterations<double, std::decay_t<decltype(Aop)>>(ctx(), method, true, cap, Aop, A, w, sites(),
+                                                                     state_.p, mirror_, L, s);
+            else
+                run_solve<double, std::decay_t<decltype(Aop)>>(ctx(), method, prec, cap, Aop, A, w, sites(), state_.p,
+                                                               mirror_, L, s, false, false, &replay_);
+        });
+        TF_CHECK(hipMemcpy(&h2, state_.p, sizeof(h2), hipMemcpyDeviceToHost));
+    }
     if (!h2.done) throw HipError("solver finished without reaching a stopping state");
     if (prec == 2) check_dic(s);
     SolveResult res;

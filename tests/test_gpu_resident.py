@@ -1,0 +1,180 @@
+"""GPU tests of the on-chip CG (csrc/cg_resident.hip).
+
+A Jacobi (or unpreconditioned) CG whose system fits the registers and LDS of
+the chip runs its iterations in one launch; TFLOWS_CG_RESIDENT=0 runs one
+launch per kernel.  The two differ only in the order in which the dot
+products are summed, so capped solves agree to rounding and converged ones
+as the parity tests of the kernel-per-phase form do with the oracle.
+
+Sizes sit at the edges of the form: one block and two, a last block of one
+slice, rows of a thread (512 threads), one-step and two-step
+synchronisation, offsets shorter and longer than a block, the locality order
+(no shared offsets), and the largest system of each kind.
+"""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def _residuals_agree(s, a, b):
+    """r = b - A x up to the rounding of its recurrence in both forms, so
+    r_a - r_b is -A (x_a - x_b) and that rounding: at most a few eps of
+    |A| |x| per iteration, 100 eps over a dozen or two."""
+    norm_a = abs(s.matrix.to_scipy()).sum(axis=1).max()
+    bound = norm_a * (np.linalg.norm(a[1] - b[1]) + 100 * 2.2e-16 * np.linalg.norm(b[1]))
+    return np.linalg.norm(a[2] - b[2]) <= bound
+
+
+def _solve(pkg, cuda, s, prec, cap, tol, method="cg"):
+    import torch
+    ds = pkg.krylov.DeviceSystem(s.matrix)
+    x = torch.zeros(s.matrix.n, dtype=torch.float64, device=cuda)
+    r = torch.from_numpy(s.b.copy()).to(cuda)
+    res = ds.solve(method, prec, x, r, cap, tol)
+    torch.cuda.synchronize()
+    ds.close()
+    return res, x.cpu().numpy(), r.cpu().numpy()
+
+
+SHAPES = {"one_slice": (4, 4, 4), "one_slice_short": (5, 3, 4), "rows_513": (3, 9, 19), "one_block_full": (16, 16, 16),
+          "two_blocks": (17, 241, 1), "last_block_short": (19, 16, 17), "line": (9000, 1, 1),
+          "blocks_64": (40, 40, 41), "blocks_64_full": (64, 64, 32), "two_step": (65, 64, 32),
+          "two_step_ragged": (67, 53, 59)}
+
+
+@pytest.mark.parametrize("shape", list(SHAPES))
+@pytest.mark.parametrize("prec", [0, 1])
+def test_capped_iterations_match(pkg, oracle, cuda, monkeypatch, shape, prec):
+    """12 iterations: the rounding of 24 sums of n terms, summed in blocks in
+    both forms (each good to about 1e-15), enters alfa and beta and grows by
+    the 12 recurrences; 1e-12 leaves two orders."""
+    s = pkg.meshgen.pressure_system(SHAPES[shape], seed=3)
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        out[mode] = _solve(pkg, cuda, s, prec, 12, 0.0)
+    a, b = out["1"], out["0"]
+    assert a[0][0] == b[0][0] == 13 and a[0][1] == b[0][1]
+    assert _rel(a[1], b[1]) <= 1e-12 and _residuals_agree(s, a, b)
+    assert a[0][2] == pytest.approx(np.linalg.norm(a[2]), rel=1e-12)
+    if s.matrix.n < 20000:
+        ref = oracle.run("cg", s.matrix, s.b, prec=prec, niter=12, tol=0.0)
+        assert _rel(a[1], ref["x"]) <= 1e-11
+
+
+@pytest.mark.parametrize("case", ["natural", "locality", "nonsymmetric", "rows_8_per_thread", "locality_largest",
+                                  "beyond"])
+def test_layouts_match(pkg, cuda, monkeypatch, case):
+    """The matrix forms a block can hold (shared offsets with symmetric and
+    with full values, columns per entry) at 20 iterations, and a system too
+    large for the form, which must give the same bits either way."""
+    mg = pkg.meshgen
+    s = {"natural": lambda: mg.pressure_system(20, seed=5),
+         "locality": lambda: mg.pressure_system((41, 37, 33), seed=6, perm_seed=2),
+         "nonsymmetric": lambda: mg.momentum_system(14, seed=7),
+         "rows_8_per_thread": lambda: mg.pressure_system((101, 99, 98), seed=8),
+         "locality_largest": lambda: mg.pressure_system((81, 80, 78), seed=9, perm_seed=3),
+         "beyond": lambda: mg.pressure_system((105, 103, 101), seed=10)}[case]()
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        out[mode] = _solve(pkg, cuda, s, 1, 20, 0.0)
+    a, b = out["1"], out["0"]
+    assert a[0][0] == b[0][0] == 21
+    if case == "beyond":
+        assert a[0] == b[0] and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+    assert _rel(a[1], b[1]) <= 1e-11 and _residuals_agree(s, a, b)
+
+
+@pytest.mark.parametrize("shape", [(2500, 1, 1), (9000, 1, 1)])
+def test_iterations_past_one_launch(pkg, cuda, monkeypatch, shape):
+    """A launch runs at most 1024 iterations; the next one goes on from its
+    x, r and p (one block, and several that read each other's p).  CG needs
+    about as many iterations as a line has cells, so both forms run past a
+    launch; each must reach the tolerance with its true residual, which the
+    recurrence's follows to the rounding of that many updates of x."""
+    s = pkg.meshgen.pressure_system(shape, seed=4)
+    A = s.matrix.to_scipy()
+    norm_a = abs(A).sum(axis=1).max()
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        (it, ini, fin), x, r = _solve(pkg, cuda, s, 1, 60000, s.tol)
+        assert 1100 < it < 60000 and fin < s.tol
+        assert np.linalg.norm(s.b - A @ x) <= s.tol + it * 2.2e-16 * norm_a * np.linalg.norm(x)
+
+
+def test_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
+    """A synchronisation that waits beyond TFLOWS_BARRIER_WAIT_MS (0: at
+    once) is given up by every block, and the solve runs one launch per
+    kernel from its inputs, to that form's bits."""
+    s = pkg.meshgen.pressure_system((40, 40, 41), seed=11)
+    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "0")
+    want = _solve(pkg, cuda, s, 1, 40, 0.0)
+    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "1")
+    whole = _solve(pkg, cuda, s, 1, 40, 0.0)
+    monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
+    got = _solve(pkg, cuda, s, 1, 40, 0.0)
+    expect = want if "gave up waiting" in capfd.readouterr().err else whole
+    assert got[0] == expect[0] and np.array_equal(got[1], expect[1]) and np.array_equal(got[2], expect[2])
+
+
+def test_two_threads(pkg, cuda):
+    """Solves from two host threads on their own streams, each a launch that
+    needs many CUs at once, give what they give alone."""
+    import torch
+    mg = pkg.meshgen
+    systems = [mg.pressure_system((67, 53, 59), seed=12), mg.pressure_system((64, 64, 32), seed=13)]
+    alone = [_solve(pkg, cuda, s, 1, 60, 0.0) for s in systems]
+    got = [[], []]
+
+    def work(q):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(5):
+                got[q].append(_solve(pkg, cuda, systems[q], 1, 60, 0.0))
+
+    ts = [threading.Thread(target=work, args=(q,)) for q in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for q in range(2):
+        assert len(got[q]) == 5
+        for g in got[q]:
+            assert g[0] == alone[q][0] and np.array_equal(g[1], alone[q][1]) and np.array_equal(g[2], alone[q][2])
+
+
+@pytest.mark.parametrize("shape", ["one_slice_short", "last_block_short", "blocks_64", "two_step_ragged", "rows_16"])
+def test_mixed_matches(pkg, cuda, monkeypatch, shape):
+    """The FP32 iterations of the reliable-update solve: both forms reach the
+    FP64 tolerance in about the same count, and their x agree as two solutions
+    with residuals below tol do (bounded here by their difference's residual)."""
+    import torch
+    mg = pkg.meshgen
+    s = mg.pressure_system((129, 127, 115) if shape == "rows_16" else SHAPES[shape], seed=14)
+    A = s.matrix.to_scipy()
+    cap = 150 if shape == "rows_16" else 3000
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        ds = pkg.krylov.DeviceSystem(s.matrix)
+        x = torch.zeros(s.matrix.n, dtype=torch.float64, device=cuda)
+        b = torch.from_numpy(s.b.copy()).to(cuda)
+        res = ds.solve_mixed_reliable(1, x, b, cap, s.tol, interval=40)
+        torch.cuda.synchronize()
+        out[mode] = (res, x.cpu().numpy())
+        ds.close()
+    a, b = out["1"], out["0"]
+    assert a[0][1] == pytest.approx(b[0][1], rel=1e-12)
+    if shape == "rows_16":             # capped: FP32 rounding over 150 iterations
+        assert a[0][0] == b[0][0] == cap + 1 and _rel(a[1], b[1]) <= 1e-4
+        return
+    assert a[0][2] < s.tol and b[0][2] < s.tol
+    assert abs(a[0][0] - b[0][0]) <= 0.05 * b[0][0] + 3
+    assert np.linalg.norm(A @ (a[1] - b[1])) <= 2 * s.tol
