@@ -75,6 +75,19 @@ class Batch {
 
    private:
     std::unique_ptr<CuShare> waiting_share(int method, int prec) const;
+    // CG of every system on the chip (cg_resident.hip): launches of as many
+    // systems as it holds at once, one after another.
+    struct ResidentWave {
+        std::vector<ResidentSystem> sys;
+        std::vector<int> index, blk_sys;   // the batch's number of each; each block's position in sys
+        int grid = 0, R = 0;
+        size_t lds = 0;
+        DevArray<ResidentSystem> d_sys;
+        DevArray<int> d_blk;
+    };
+    bool resident_waves();               // builds waves_; false: this batch's rows or sizes do not allow it
+    bool run_resident(int prec, const KrylovVectors<double>& w, const std::vector<SolverState>& init,
+                      const std::function<void()>& prepare, std::vector<SolverState>& out);
     struct Key {
         int bits, method, prec;
         bool operator<(const Key& o) const {
@@ -164,6 +177,10 @@ class Batch {
     // stay resident from one iteration to the next while the group runs
     double mall_budget_ = 192.0 * 1024 * 1024;
     bool persistent_ok_ = true;
+    int resident_ = 2;                   // 2: not tried; 1: waves_ built; 0: kernel forms only
+    std::vector<std::unique_ptr<ResidentWave>> waves_;
+    DevArray<uint64_t> res_posts_;       // kPostTotal words per system of several blocks
+    uint32_t res_tag_ = 0;
     DevArray<int> bar_, pfault_;       // barrier counters (one per system) and the fault word of the persistent form
     uint64_t wait_ticks_ = 0;
     hipEvent_t ev_[5] = {};            // pacing (2), tuner timing (2), join

@@ -823,10 +823,167 @@ static void check_method(int method, int prec) {
     if (prec < 0 || prec > 2) throw std::invalid_argument("prec must be 0, 1 or 2");
 }
 
+// Each system's column offsets, when its rows are short, ascend and use few
+// of them (a box in natural order), and the shares of the chip: every system
+// takes blocks of at most kMaxRows rows; systems are dealt out, largest
+// first, to as few launches as hold all blocks at once, and a launch's blocks
+// are then made as small as its CUs allow.
+bool Batch::resident_waves() {
+    if (resident_ != 2) return resident_ == 1;
+    resident_ = 0;
+    constexpr int kMaxRows = resident_rows_per_thread<double>(false) * kResThreads;
+    const std::vector<int>&rp = sys_->host_rowptr(), &cl = sys_->host_col();
+    std::vector<std::vector<int>> offsets(k_);
+    for (int q = 0; q < k_; ++q) {
+        std::vector<int>& of = offsets[q];
+        for (int i = roff_[q]; i < roff_[q + 1]; ++i)
+            for (int e = rp[i]; e < rp[i + 1]; ++e) {
+                if (e > rp[i] && cl[e] <= cl[e - 1]) return false;
+                const int d = cl[e] - i;
+                if (std::find(of.begin(), of.end(), d) != of.end()) continue;
+                of.push_back(d);
+                if ((int)of.size() > window_slots<double>()) return false;
+            }
+        std::sort(of.begin(), of.end());
+    }
+    const int cus = resident_blocks();
+    if (cus <= 0) return false;
+    auto blocks = [&](int q, int rows) {
+        int nb = (roff_[q + 1] - roff_[q] + rows - 1) / rows;
+        if (nb > kWave) nb = (nb + kNumXcd - 1) / kNumXcd * kNumXcd;   // two-step synchronisation
+        return nb;
+    };
+    int64_t total = 0;
+    std::vector<int> order(k_);
+    for (int q = 0; q < k_; ++q) {
+        order[q] = q;
+        total += blocks(q, kMaxRows);
+        if (blocks(q, kMaxRows) > cus) return false;
+    }
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int b) { return roff_[a + 1] - roff_[a] > roff_[b + 1] - roff_[b]; });
+    for (int nw = (int)((total + cus - 1) / cus);; ++nw) {
+        std::vector<std::vector<int>> deal(nw);
+        std::vector<int> used(nw, 0);
+        bool fits = true;
+        for (int q : order) {
+            const int at = (int)(std::min_element(used.begin(), used.end()) - used.begin());
+            used[at] += blocks(q, kMaxRows);
+            fits = fits && used[at] <= cus;
+            deal[at].push_back(q);
+        }
+        if (!fits) continue;             // ends: one launch per system holds every system
+        for (const auto& systems : deal) {
+            auto need = [&](int rows) {
+                int64_t n = 0;
+                for (int q : systems) n += blocks(q, rows);
+                return n;
+            };
+            int rows = 2 * kResThreads;
+            while (rows < kMaxRows && need(rows) > cus) rows += kSlice;
+            std::unique_ptr<ResidentWave> wv(new ResidentWave);
+            for (int q : systems) {
+                ResidentSystem s{};
+                const int n = roff_[q + 1] - roff_[q];
+                s.grid = blocks(q, rows);
+                s.blk0 = wv->grid;
+                wv->grid += s.grid;
+                ResidentShape sh;
+                sh.grid = s.grid;
+                sh.rows = ((n + s.grid - 1) / s.grid + kSlice - 1) / kSlice * kSlice;
+                if (!window_shape<double>(sh, offsets[q], s.w)) return false;
+                s.a.n = n;
+                s.a.rows = sh.rows;
+                wv->R = std::max(wv->R, (sh.rows + kResThreads - 1) / kResThreads);
+                wv->blk_sys.insert(wv->blk_sys.end(), s.grid, (int)wv->sys.size());
+                wv->sys.push_back(s);
+                wv->index.push_back(q);
+            }
+            for (auto& s : wv->sys) {
+                s.w.lds = batch_window_lds(s, wv->R);
+                wv->lds = std::max(wv->lds, s.w.lds);
+            }
+            if (wv->lds > kResLdsBytes) return false;
+            waves_.push_back(std::move(wv));
+        }
+        break;
+    }
+    resident_ = 1;
+    return true;
+}
+
+bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::vector<SolverState>& init,
+                         const std::function<void()>& prepare, std::vector<SolverState>& out) {
+    // the set-up and the first stopping test of the kernel forms
+    const int G = std::min(gmax_, std::max(round8(k_), 2048));
+    TF_CHECK(hipStreamSynchronize(bs_));
+    build_maps(std::vector<char>(k_, 1), G);
+    upload_maps(bs_);
+    prepare();
+    TF_CHECK(hipMemcpyAsync(st_.p, init.data(), sizeof(SolverState) * k_, hipMemcpyHostToDevice, bs_));
+    const Csr<double> A = sys_->csr();
+    const Sites<double> S = Sites<double>::carve(partials_.p, G);
+    const BatchCtx c0 = ctx(1, false);
+    start_solve<double, Csr<double>>(c0, 0, prec, A, A, w, S, st_.p, nullptr, &kNoLevels, bs_, false, false);
+    launch_check(c0, 1, S, st_.p, nullptr, bs_);
+    const size_t words = (size_t)kPostTotal * k_;
+    if (!res_posts_.p || res_tag_ > (1u << 30)) {
+        res_posts_.ensure(words);
+        TF_CHECK(hipMemsetAsync(res_posts_.p, 0, sizeof(uint64_t) * words, bs_));
+        res_tag_ = 0;
+    }
+    bool ok = true;
+    out.resize(k_);
+    for (auto& wv : waves_) {
+        for (size_t j = 0; j < wv->sys.size(); ++j) {
+            ResidentSystem& s = wv->sys[j];
+            const int q = wv->index[j], r0 = roff_[q];
+            s.A = CsrRows{s.a.n, r0, A.rowptr + r0, A.col, A.val};
+            s.a.chunk = kResChunk;
+            s.a.x = w.x + r0;
+            s.a.r = w.r1 + r0;
+            s.a.p = w.p + r0;
+            s.a.z = w.u1 + r0;
+            s.a.D = w.D + r0;
+            s.a.slotB = res_posts_.p + (size_t)kPostTotal * q;
+            s.a.slotC = s.a.slotB + kPostTotal / 2;
+            s.a.wait_ticks = wait_ticks_;
+            s.a.st = st_.p + q;
+        }
+        wv->d_sys.ensure(wv->sys.size());
+        wv->d_blk.ensure(wv->blk_sys.size());
+        TF_CHECK(hipMemcpyAsync(wv->d_sys.p, wv->sys.data(), sizeof(ResidentSystem) * wv->sys.size(),
+                                hipMemcpyHostToDevice, bs_));
+        TF_CHECK(hipMemcpyAsync(wv->d_blk.p, wv->blk_sys.data(), sizeof(int) * wv->blk_sys.size(),
+                                hipMemcpyHostToDevice, bs_));
+    }
+    for (;;) {
+        for (auto& wv : waves_) {
+            ok = ok && launch_cg_window_batch(wv->d_sys.p, wv->d_blk.p, wv->grid, wv->R, wv->lds, res_tag_, bs_);
+            res_tag_ += resident_tags(kResChunk);
+        }
+        TF_CHECK(hipGetLastError());
+        TF_CHECK(hipMemcpyAsync(out.data(), st_.p, sizeof(SolverState) * k_, hipMemcpyDeviceToHost, bs_));
+        TF_CHECK(hipStreamSynchronize(bs_));
+        bool all = true;
+        for (const auto& h : out) {
+            all = all && h.done;
+            ok = ok && !h.fault;
+        }
+        if (!ok) break;
+        if (all) return true;
+    }
+    resident_ = 0;
+    std::fprintf(stderr, "libtflows_krylov: an on-chip batch launch gave up waiting (TFLOWS_BARRIER_WAIT_MS); the "
+                         "batch now runs its kernel forms\n");
+    std::fflush(stderr);
+    return false;
+}
+
 // The device's CUs, where the launches of a solve may wait for each other's
 // blocks (DIC sweeps, the persistent form).
 std::unique_ptr<CuShare> Batch::waiting_share(int method, int prec) const {
-    const bool waits = prec == 2 ? sys_->dic_form() >= 2 : method == 0 && persistent_ok_;
+    const bool waits = prec == 2 ? sys_->dic_form() >= 2 : method == 0;
     return std::unique_ptr<CuShare>(waits ? new CuShare(-1) : nullptr);
 }
 
@@ -850,10 +1007,14 @@ void Batch::solve(int method, int prec, double* x, double* r1, const int* cap, c
     };
     const Csr<double> A = sys_->csr();
     std::vector<SolverState> out;
-    sys_->with_op64(bs_, [&](const auto& Aop) {
-        run<double, std::decay_t<decltype(Aop)>>(64, method, prec, Aop, A, w, partials_.p, st_.p, hm_, init, false,
-                                                 false, prepare, out);
-    });
+    // on the chip, unless a form, launch shape or grouping is fixed
+    const bool chosen = form_ || groups_ || fixed_.grid || fixed_.lanes || fixed_.chunk;
+    if (method != 0 || prec == 2 || chosen || !cg_resident_enabled() || !resident_waves() ||
+        !run_resident(prec, w, init, prepare, out))
+        sys_->with_op64(bs_, [&](const auto& Aop) {
+            run<double, std::decay_t<decltype(Aop)>>(64, method, prec, Aop, A, w, partials_.p, st_.p, hm_, init, false,
+                                                     false, prepare, out);
+        });
     scatter_out(w.x, x);
     scatter_out(w.r1, r1);
     TF_CHECK(hipStreamSynchronize(bs_));

@@ -29,6 +29,8 @@ struct ResidentShape {
     int grid = 0, rows = 0;
 };
 ResidentShape resident_shape(int n, int rows_per_thread);
+// the most blocks of a launch: one per CU
+int resident_blocks();
 
 // rows of a thread that the registers hold: FP64 8 (14 of 256 registers per
 // row's values) and FP32 16 of a shared-offset matrix, half where every entry
@@ -95,6 +97,21 @@ struct ResidentArgs {
     uint64_t wait_ticks;
     SolverState* st;       // its `fault` word ends every wait of the launch
 };
+// CSR rows of one system of a block-diagonal matrix (rowptr at its first
+// row, columns counted over the whole matrix)
+struct CsrRows {
+    int n, row0;
+    const int* __restrict__ rowptr;
+    const int* __restrict__ col;
+    const double* __restrict__ val;
+};
+// One system of a batched launch: blocks blk0 .. blk0 + grid - 1.
+struct ResidentSystem {
+    CsrRows A;
+    ResidentArgs<double> a;
+    WindowShape w;
+    int grid, blk0;
+};
 // synchronisations a launch of `chunk` iterations may number
 inline uint32_t resident_tags(int chunk) { return 3u * (uint32_t)chunk + 3u; }
 
@@ -126,5 +143,9 @@ template <typename Op, typename T>
 bool launch_cg_stream(const Op& A, const ResidentArgs<T>& a, int grid, hipStream_t s);
 template <typename Op, typename T>
 bool launch_cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, int grid, hipStream_t s);
+// LDS of system s in a launch of R rows per thread (the most of any system)
+size_t batch_window_lds(const ResidentSystem& s, int R);
+bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, uint32_t tag,
+                            hipStream_t s);
 
 }  // namespace tflows

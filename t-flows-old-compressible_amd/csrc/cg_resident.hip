@@ -384,6 +384,26 @@ __device__ __forceinline__ void load_row(const Op& A, int row, bool live, const 
     }
 }
 
+// The same from the CSR arrays (a system of a block-diagonal batch): every
+// column offset of the row is one of w.offset.
+template <bool SHARED, typename T>
+__device__ __forceinline__ void load_row(const CsrRows& A, int row, bool live, const WindowShape& w, int, int,
+                                         RowSlots<T, SHARED>& s) {
+    static_assert(SHARED, "rows of known offsets");
+    constexpr int N = RowSlots<T, SHARED>::N;
+#pragma unroll
+    for (int j = 0; j < N; ++j) s.a[j] = T(0);
+    if (!live) return;
+    const int e1 = A.rowptr[row + 1];
+    for (int e = A.rowptr[row]; e < e1; ++e) {
+        const int d = A.col[e] - A.row0 - row;
+        const T v = A.val[e];
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (j < w.nslots && d == w.offset[j]) s.a[j] = v;
+    }
+}
+
 // Products added to 0 in CSR order (CG.f90:193-199), or the terms of the
 // difference form, gathered from LDS; `off` is an opaque 0.  Row k of a thread lies k * kResThreads above its first, an
 // immediate offset of the LDS reads.
@@ -574,8 +594,9 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
 // SHARED: shared-offset matrix, the halo being `lo` rows either side and the
 // far regions of w; else the halo is the window of columns the block reaches
 // (deps).  LDS: halo below, own rows, halo above, far regions.
-template <typename Op, bool SHARED, int R, bool MIXED, typename T = typename OpValue<Op>::type>
-__global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T> a, WindowShape w) {
+template <typename Op, bool SHARED, int R, bool MIXED, typename T>
+__device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, const int G,
+                                          const int blk) {
     extern __shared__ __align__(16) char res_lds[];
     __shared__ T sm[2 * kResThreads];
     __shared__ int s_fail, s_done;
@@ -585,7 +606,6 @@ __global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T>
         s_fail = 0;
         s_done = st->done | st->suspend | st->fault;
     }
-    const int G = gridDim.x, blk = logical_block();
     const int rb = min(blk * a.rows, a.n), nloc = min(a.n - rb, a.rows);
     const bool lead = blk == 0 && tid == 0;
     const double tol = st->tol;
@@ -778,6 +798,23 @@ __global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T>
     }
 }
 
+template <typename Op, bool SHARED, int R, bool MIXED, typename T = typename OpValue<Op>::type>
+__global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T> a, WindowShape w) {
+    cg_window<Op, SHARED, R, MIXED, T>(A, a, w, gridDim.x, logical_block());
+}
+
+// Many systems in one launch: each has its own blocks, posts and state, and
+// goes its own way (a system that has stopped, or whose blocks stop early,
+// leaves the others alone).
+template <int R>
+__global__ __launch_bounds__(kResThreads) void k_cg_window_batch(const ResidentSystem* __restrict__ sys,
+                                                                 const int* __restrict__ blk_sys, uint32_t tag) {
+    const ResidentSystem& s = sys[blk_sys[blockIdx.x]];
+    ResidentArgs<double> a = s.a;
+    a.tag = tag;
+    cg_window<CsrRows, true, R, false, double>(s.A, a, s.w, s.grid, (int)blockIdx.x - s.blk0);
+}
+
 // Smallest and largest column of each block's rows.
 __global__ __launch_bounds__(kBlock) void k_resident_deps(int n, int rows, const int* __restrict__ rowptr,
                                                           const int* __restrict__ col, int* __restrict__ deps) {
@@ -827,15 +864,20 @@ uint64_t resident_wait_ticks() {
     return (uint64_t)khz * (uint64_t)(ms < 0 ? 0 : ms);
 }
 
+int resident_blocks() {
+    const int cus = std::min(device_cus(), kResMaxBlocks);
+    return cus >= kNumXcd ? cus / kNumXcd * kNumXcd : cus;   // whole shares of the XCDs
+}
+
 ResidentShape resident_shape(int n, int rows_per_thread) {
     ResidentShape r;
-    const int cus = std::min(device_cus(), kResMaxBlocks);
+    const int cus = resident_blocks();
     if (n <= 0 || cus <= 0) return r;
     int grid = 1;
     if (n > kResOneBlockRows) {
         grid = std::min(cus, (n + kResMinRows - 1) / kResMinRows);
         if (grid > kWave && n <= kWave * 2 * kResMinRows) grid = kWave;
-        if (grid >= kNumXcd) grid = grid / kNumXcd * kNumXcd;   // whole shares of the XCDs
+        if (grid >= kNumXcd) grid = grid / kNumXcd * kNumXcd;
     }
     const int64_t rows = (((int64_t)n + grid - 1) / grid + kSlice - 1) / kSlice * kSlice;
     if (rows > (int64_t)rows_per_thread * kResThreads) return r;
@@ -969,6 +1011,27 @@ bool launch_cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& 
     return A.soff ? launch_window<true>(std::integral_constant<int, 1>{}, R, A, a, w, grid, s)
                   : launch_window<false>(std::integral_constant<int, 1>{}, R, A, a, w, grid, s);
 }
+template <int N>
+static bool launch_batch(std::integral_constant<int, N>, int R, int grid, size_t lds, const ResidentSystem* sys,
+                         const int* blk_sys, uint32_t tag, hipStream_t s) {
+    if constexpr (N > resident_rows_per_thread<double>(false)) {
+        return false;
+    } else {
+        if (R <= N) return launch_resident(k_cg_window_batch<N>, grid, lds, s, sys, blk_sys, tag);
+        return launch_batch(std::integral_constant<int, window_kernel_rows(N + 1)>{}, R, grid, lds, sys, blk_sys, tag,
+                            s);
+    }
+}
+size_t batch_window_lds(const ResidentSystem& s, int R) {
+    const int K = window_kernel_rows(std::max(R, 2));
+    return sizeof(double) * (2 * (size_t)s.w.lo + (size_t)s.w.nfar * s.a.rows +
+                             (size_t)K * kResThreads * (window_d_in_lds<double>(K) ? 2 : 1));
+}
+bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, uint32_t tag,
+                            hipStream_t s) {
+    return launch_batch(std::integral_constant<int, 2>{}, R, grid, lds, sys, blk_sys, tag, s);
+}
+
 template bool launch_cg_window<Sell<double>, double>(const Sell<double>&, const ResidentArgs<double>&,
                                                      const WindowShape&, int, hipStream_t);
 template bool launch_cg_window<DiffSell32, float>(const DiffSell32&, const ResidentArgs<float>&, const WindowShape&,

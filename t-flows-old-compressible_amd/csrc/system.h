@@ -334,6 +334,9 @@ class System {
     const int* rowptr() const { return rowptr_.p; }
     const int* col() const { return col_.p; }
     const int* dia() const { return dia_.p; }
+    // the 0-based pattern on the host (the caller's order)
+    const std::vector<int>& host_rowptr() const { return h_rowptr_; }
+    const std::vector<int>& host_col() const { return h_col_; }
 
     Sites<double> sites();
     KrylovVectors<double> vectors(double* x, double* r1);

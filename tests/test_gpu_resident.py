@@ -178,3 +178,72 @@ def test_mixed_matches(pkg, cuda, monkeypatch, shape):
     assert a[0][2] < s.tol and b[0][2] < s.tol
     assert abs(a[0][0] - b[0][0]) <= 0.05 * b[0][0] + 3
     assert np.linalg.norm(A @ (a[1] - b[1])) <= 2 * s.tol
+
+
+def _batch(pkg, cuda, systems, form, caps, tols, prec=1, b=None):
+    import torch
+    B = pkg.krylov.DeviceBatch([s.matrix for s in systems])
+    B.set_form(form)
+    x = torch.zeros(B.rows, dtype=torch.float64, device=cuda)
+    r = torch.from_numpy(np.concatenate([s.b for s in systems] if b is None else b)).to(cuda)
+    out = []
+    for _ in range(2):                 # twice: the posts and the state carry over
+        xx, rr = x.clone(), r.clone()
+        res = B.solve("cg", prec, xx, rr, caps, tols, fin_in=np.full(len(systems), 0.5))
+        torch.cuda.synchronize()
+        out.append((res, [v.cpu().numpy() for v in B.split(xx)], [v.cpu().numpy() for v in B.split(rr)]))
+    B.close()
+    return out
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_batch_matches_kernel_form(pkg, cuda, prec):
+    """Systems of one row to several blocks, in one launch: converged, capped
+    and early-exit ones, against one launch per kernel (form 1)."""
+    import scipy.sparse as sp
+    mg = pkg.meshgen
+    one = mg.LinearSystem(mg.from_scipy(sp.csr_matrix(np.array([[4.0]]))), np.array([2.0]), np.zeros(1), 1e-8, 1, 100, {})
+    shapes = [(7, 5, 3), (16, 16, 16), (17, 241, 1), (40, 40, 41), (13, 11, 17), (9000, 1, 1), (64, 64, 32)]
+    systems = [mg.pressure_system(sh, seed=20 + q) for q, sh in enumerate(shapes)] + [one]
+    caps = np.array([3000, 12, 12, 3000, 3000, 15, 3000, 10], np.int32)
+    tols = np.array([s.tol for s in systems])
+    b = [s.b.copy() for s in systems]
+    b[4][:] = 0.0                      # ||b|| < tol: the early exit
+    got = _batch(pkg, cuda, systems, 0, caps, tols, prec, b)
+    ref = _batch(pkg, cuda, systems, 1, caps, tols, prec, b)[0]
+    for a in got:
+        assert np.array_equal(a[0]["niter"], got[0][0]["niter"])
+        for q, s in enumerate(systems):
+            assert np.array_equal(a[1][q], got[0][1][q]) and np.array_equal(a[2][q], got[0][2][q])
+            assert abs(int(a[0]["niter"][q]) - int(ref[0]["niter"][q])) <= 1, q
+            if a[0]["niter"][q] <= caps[q] and q != 4:
+                assert a[0]["fin_res"][q] < tols[q]
+                assert np.linalg.norm(s.b - s.matrix.to_scipy() @ a[1][q]) < 10 * tols[q]
+            elif q != 4:               # capped after a dozen iterations
+                assert _rel(a[1][q], ref[1][q]) <= 1e-12
+        assert a[0]["niter"][4] == 0 and a[0]["fin_res"][4] == 0.5 and not np.any(a[1][4])
+
+
+def test_batch_of_several_launches(pkg, cuda):
+    """More rows than the chip holds: the systems are dealt out to several
+    launches."""
+    mg = pkg.meshgen
+    systems = [mg.pressure_system((61, 60, 59), seed=30 + q) for q in range(6)] + [mg.pressure_system(9, seed=40)]
+    caps, tols = np.full(7, 12, np.int32), np.zeros(7)
+    a, ref = _batch(pkg, cuda, systems, 0, caps, tols)[0], _batch(pkg, cuda, systems, 1, caps, tols)[0]
+    for q in range(7):
+        assert a[0]["niter"][q] == ref[0]["niter"][q] == 13
+        assert _rel(a[1][q], ref[1][q]) <= 1e-12
+
+
+def test_batch_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
+    mg = pkg.meshgen
+    systems = [mg.pressure_system((40, 40, 41), seed=50), mg.pressure_system((41, 39, 38), seed=51)]
+    caps, tols = np.full(2, 30, np.int32), np.zeros(2)
+    whole = _batch(pkg, cuda, systems, 0, caps, tols)[0]
+    monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
+    got = _batch(pkg, cuda, systems, 0, caps, tols)[0]
+    gave_up = "gave up waiting" in capfd.readouterr().err
+    for q in range(2):
+        assert got[0]["niter"][q] == 31
+        assert _rel(got[1][q], whole[1][q]) <= 1e-11 if gave_up else np.array_equal(got[1][q], whole[1][q])
