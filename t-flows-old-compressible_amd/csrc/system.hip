@@ -1280,7 +1280,9 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
         const bool window = !csr_rows && window_of(shape, sell64(s), sell64_width_, sell64_offsets_, win);
         auto launch = [&](const ResidentArgs<double>& a) {
             if (window) return launch_cg_window(sell64(s), a, win, shape.grid, s);
-            return csr_rows ? launch_cg_stream(A, a, shape.grid, s) : launch_cg_stream(sell64(s), a, shape.grid, s);
+            // (k_cg_stream reads columns, which a shared-offset copy does not hold)
+            return csr_rows || sell64(s).soff ? launch_cg_stream(A, a, shape.grid, s)
+                                              : launch_cg_stream(sell64(s), a, shape.grid, s);
         };
         resident = run_resident(shape, sp, launch, w, state_.p, h, h2, s);
         if (!resident) {

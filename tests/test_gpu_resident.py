@@ -93,6 +93,28 @@ def test_layouts_match(pkg, cuda, monkeypatch, case):
     assert _rel(a[1], b[1]) <= 1e-11 and _residuals_agree(s, a, b)
 
 
+def test_shared_offsets_beyond_the_window(pkg, oracle, cuda, monkeypatch):
+    """Two boxes of different lines in one system: each slice's offsets are
+    shared, but the system has more of them than a block's halo allows, so
+    the rows are read from the CSR arrays every iteration."""
+    import scipy.sparse as sp
+    mg = pkg.meshgen
+    parts = [mg.pressure_system((16, 4, 8), seed=15), mg.pressure_system((13, 7, 9), seed=16),
+             mg.pressure_system((40, 40, 41), seed=17)]
+    for some in (parts[:2], [parts[0], parts[2]]):
+        A = sp.block_diag([q.matrix.to_scipy() for q in some], format="csr")
+        s = mg.LinearSystem(mg.from_scipy(A), np.concatenate([q.b for q in some]), np.zeros(A.shape[0]), 1e-8, 1, 100, {})
+        out = {}
+        for mode in ("1", "0"):
+            monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+            ds = pkg.krylov.DeviceSystem(s.matrix)
+            assert ds.fp64_layout()["shared"]
+            ds.close()
+            out[mode] = _solve(pkg, cuda, s, 1, 12, 0.0)
+        assert out["1"][0][0] == out["0"][0][0] == 13
+        assert _rel(out["1"][1], out["0"][1]) <= 1e-12 and _residuals_agree(s, out["1"], out["0"])
+
+
 @pytest.mark.parametrize("shape", [(2500, 1, 1), (9000, 1, 1)])
 def test_iterations_past_one_launch(pkg, cuda, monkeypatch, shape):
     """A launch runs at most 1024 iterations; the next one goes on from its
