@@ -113,7 +113,7 @@ struct ResidentSystem {
     int grid, blk0;
 };
 // synchronisations a launch of `chunk` iterations may number
-inline uint32_t resident_tags(int chunk) { return 3u * (uint32_t)chunk + 3u; }
+inline uint32_t resident_tags(int chunk) { return 4u * (uint32_t)chunk + 4u; }
 
 // TFLOWS_CG_RESIDENT=0, or an explicit kernel-per-phase form (TFLOWS_CG_FORM,
 // TFLOWS_CG_CARRY), turns the on-chip CG off (read at every solve)
@@ -143,6 +143,10 @@ template <typename Op, typename T>
 bool launch_cg_stream(const Op& A, const ResidentArgs<T>& a, int grid, hipStream_t s);
 template <typename Op, typename T>
 bool launch_cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, int grid, hipStream_t s);
+// CGS: rows of a thread (seven vectors and the matrix rows in registers)
+constexpr int kCgsRows = 4;
+bool launch_cgs_window(const Sell<double>& A, const ResidentArgs<double>& a, const WindowShape& w, const double* r2,
+                       double* q, double* u2, int grid, hipStream_t s);
 // LDS of system s in a launch of R rows per thread (the most of any system)
 size_t batch_window_lds(const ResidentSystem& s, int R);
 bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, uint32_t tag,

@@ -224,6 +224,29 @@ __device__ __forceinline__ bool resident_sum(int tid, T (&v)[NV], uint64_t* slot
     return *s_fail == 0;
 }
 
+// Synchronisation A: this block's published rows have reached memory, and
+// those of the blocks its columns reach (alo .. ahi) have.  False when the
+// wait was given up (the whole block agrees).
+__device__ __forceinline__ bool neighbour_sync(uint32_t* flags, int blk, int alo, int ahi, uint32_t tag,
+                                               const Waiter& wt, int* s_fail) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    const int tid = threadIdx.x;
+    if (tid == 0) __hip_atomic_store(flags + blk, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int b = alo + tid;
+    if (b <= ahi && b != blk) {
+        unsigned polls = 0;
+        uint64_t t0 = 0;
+        while ((int)(__hip_atomic_load(flags + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - tag) < 0)
+            if (!wt.keep_waiting(polls, t0)) {
+                *s_fail = 1;
+                break;
+            }
+    }
+    __syncthreads();
+    return *s_fail == 0;
+}
+
 // A vector of other blocks' values, read W (16 bytes of) rows at a time with
 // device-coherent loads (the same cache policy as the atomic loads above: a
 // wider access needs no atomicity, since the rows of a granule are complete
@@ -426,27 +449,7 @@ __device__ __forceinline__ T row_sum(const RowSlots<T, SHARED>& s, int k, int ow
     return acc;
 }
 
-// Rows of any width, read from memory slot by slot.
-template <typename T>
-__device__ __forceinline__ T stream_row(const Sell<T>& A, int row, const ResGather<T>& g) {
-    const int sl = __builtin_amdgcn_readfirstlane(row / kSlice);
-    const int b = A.off[sl] + row - sl * kSlice;
-    const int w = (A.off[sl + 1] - A.off[sl]) / kSlice;
-    T acc = T(0);
-#pragma unroll 4
-    for (int j = 0; j < w; ++j) {
-        int c = -1;
-        if (A.dc) {
-            const short d = A.dc[b + j * kSlice];
-            if (d != kPad16) c = row + (int)d;
-        } else {
-            c = A.col[b + j * kSlice];
-        }
-        const T sum = acc + A.val[b + j * kSlice] * g(c >= 0, c);
-        acc = c >= 0 ? sum : acc;
-    }
-    return acc;
-}
+// A row of any length, read from memory.
 template <typename T>
 __device__ __forceinline__ T stream_row(const Csr<T>& A, int row, const ResGather<T>& g) {
     T acc = T(0);
@@ -537,23 +540,10 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
             if (G > 1 && l < nloc) coherent_store(a.p + rb + l, p);
         }
         if (G > 1) {
-            ++tag;
-            __builtin_amdgcn_s_waitcnt(0);               // this wave's p stores have reached memory
+            if (!neighbour_sync(a.flags, blk, alo, ahi, ++tag, wt, &s_fail)) return;
+        } else {
             __syncthreads();
-            if (tid == 0) __hip_atomic_store(a.flags + blk, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int b = alo + tid;
-            if (b <= ahi && b != blk) {
-                unsigned polls = 0;
-                uint64_t t0 = 0;
-                while ((int)(__hip_atomic_load(a.flags + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - tag) < 0)
-                    if (!wt.keep_waiting(polls, t0)) {
-                        s_fail = 1;
-                        break;
-                    }
-            }
         }
-        __syncthreads();
-        if (s_fail) return;
         T pq[1] = {T(0)};
 #pragma unroll
         for (int k = 0; k < R; ++k) {
@@ -588,6 +578,49 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
             st->done = 1;
             st->niter_out = niter;
         }
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ HaloRun far_run(const WindowShape& w, int rb, int rows, int q) {
+    return HaloRun{w.farbase + q * rows, rb + w.far[q], q < w.nfar ? rows / CoherentVec<T>::W : 0};
+}
+
+// The halo's p = z + beta p (z when first): every run's loads in flight
+// together, R rows per thread.
+template <bool SHARED, int R, typename T>
+__device__ __forceinline__ void halo_update(int t, const CoherentVec<T>& zin, T* lp, const HaloRun& below,
+                                            const HaloRun& above, const WindowShape& w, int rb, int rows, bool first,
+                                            T beta) {
+    constexpr int NF = (R + CoherentVec<T>::W - 1) / CoherentVec<T>::W;   // granules of a far run per thread
+    if constexpr (SHARED) {
+        auto far = [&](int q) { return far_run<T>(w, rb, rows, q); };
+        HaloLoad<T, NF> f0, f1;
+        HaloLoad<T, 1> n0, n1;
+        f0.load(t, zin, far(0));
+        f1.load(t, zin, far(1));
+        n0.load(t, zin, below);
+        n1.load(t, zin, above);
+        f0.apply(t, zin, lp, far(0), first, beta);
+        f1.apply(t, zin, lp, far(1), first, beta);
+        n0.apply(t, zin, lp, below, first, beta);
+        n1.apply(t, zin, lp, above, first, beta);
+        n0.rest(t, zin, lp, below, first, beta);
+        n1.rest(t, zin, lp, above, first, beta);
+        if (w.nfar > 2) {
+            f0.load(t, zin, far(2));
+            f1.load(t, zin, far(3));
+            f0.apply(t, zin, lp, far(2), first, beta);
+            f1.apply(t, zin, lp, far(3), first, beta);
+        }
+    } else {
+        HaloLoad<T, 4> n0, n1;
+        n0.load(t, zin, below);
+        n1.load(t, zin, above);
+        n0.apply(t, zin, lp, below, first, beta);
+        n1.apply(t, zin, lp, above, first, beta);
+        n0.rest(t, zin, lp, below, first, beta);
+        n1.rest(t, zin, lp, above, first, beta);
     }
 }
 
@@ -652,7 +685,6 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
     constexpr int W = 16 / (int)sizeof(T);
     const CoherentVec<T> zin(a.z, a.n);
     const HaloRun below{0, rb - lo, lo / W}, above{lo + a.rows, rb + a.rows, hi / W};
-    auto far = [&](int q) { return HaloRun{w.farbase + q * a.rows, rb + w.far[q], q < w.nfar ? a.rows / W : 0}; };
     auto first_p = [&](const HaloRun& h) {
         for (int e = tid; it0 > 0 && e < h.count * W; e += kResThreads)
             if (h.row + e >= 0 && h.row + e < a.n) lp[h.at + e] = a.p[h.row + e];
@@ -660,7 +692,7 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
     first_p(below);
     first_p(above);
     if (SHARED)
-        for (int q = 0; q < w.nfar; ++q) first_p(far(q));
+        for (int q = 0; q < w.nfar; ++q) first_p(far_run<T>(w, rb, a.rows, q));
     double err64 = 0.0;
     if (MIXED) {                    // the FP64 norm of the replacement before this launch (site E)
         __shared__ double sm64[kResThreads];
@@ -718,37 +750,7 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
         const bool first = it == 0;
         const T beta = first ? T(0) : rho / rho_old;                // CG.f90:183
         rho_old = rho;
-        if (G > 1) {                                 // the halo's p, every run's loads in flight together
-            constexpr int NF = (R + W - 1) / W;      // granules of a far run per thread
-            if constexpr (SHARED) {
-                HaloLoad<T, NF> f0, f1;
-                HaloLoad<T, 1> n0, n1;
-                f0.load(t, zin, far(0));
-                f1.load(t, zin, far(1));
-                n0.load(t, zin, below);
-                n1.load(t, zin, above);
-                f0.apply(t, zin, lp, far(0), first, beta);
-                f1.apply(t, zin, lp, far(1), first, beta);
-                n0.apply(t, zin, lp, below, first, beta);
-                n1.apply(t, zin, lp, above, first, beta);
-                n0.rest(t, zin, lp, below, first, beta);
-                n1.rest(t, zin, lp, above, first, beta);
-                if (w.nfar > 2) {
-                    f0.load(t, zin, far(2));
-                    f1.load(t, zin, far(3));
-                    f0.apply(t, zin, lp, far(2), first, beta);
-                    f1.apply(t, zin, lp, far(3), first, beta);
-                }
-            } else {
-                HaloLoad<T, 4> n0, n1;
-                n0.load(t, zin, below);
-                n1.load(t, zin, above);
-                n0.apply(t, zin, lp, below, first, beta);
-                n1.apply(t, zin, lp, above, first, beta);
-                n0.rest(t, zin, lp, below, first, beta);
-                n1.rest(t, zin, lp, above, first, beta);
-            }
-        }
+        if (G > 1) halo_update<SHARED, R>(t, zin, lp, below, above, w, rb, a.rows, first, beta);
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             const int l = k * kResThreads + t;
@@ -801,6 +803,174 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
 template <typename Op, bool SHARED, int R, bool MIXED, typename T = typename OpValue<Op>::type>
 __global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T> a, WindowShape w) {
     cg_window<Op, SHARED, R, MIXED, T>(A, a, w, gridDim.x, logical_block());
+}
+
+// CGS (Process/CGS.f90:112-334) in the same form: x, r, the shadow r2, q, u1,
+// u2, D and the matrix rows in registers, the vector of the next product
+// (own rows and halo) in LDS.  Its two products an iteration act on vectors
+// that need the scalar just reduced and a division by D, so each is
+// published after that (synchronisation A):
+//
+//   C  ||r||^2, rho = (r, r2)  -> stopping test, beta; u1, u2; u2 / D published
+//   A  -> halo, v = A (u2 / D)
+//   B  (r2, v)                 -> alfa; q; w = (u1 + q) / D published
+//   A  -> halo, x += alfa w, r -= alfa A w
+//
+// qg, u2g carry q and u2 from launch to launch.
+template <typename Op, bool SHARED, int R, typename T = typename OpValue<Op>::type>
+__global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T> a, WindowShape w,
+                                                            const T* __restrict__ shadow, T* __restrict__ qg,
+                                                            T* __restrict__ u2g) {
+    extern __shared__ __align__(16) char res_lds[];
+    __shared__ T sm[2 * kResThreads];
+    __shared__ int s_fail, s_done;
+    SolverState* st = a.st;
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        s_fail = 0;
+        s_done = st->done | st->fault;
+    }
+    const int G = gridDim.x, blk = logical_block();
+    const int rb = min(blk * a.rows, a.n), nloc = min(a.n - rb, a.rows);
+    const bool lead = blk == 0 && tid == 0;
+    const double tol = st->tol;
+    const int cap = st->cap, it0 = st->it;
+    T rho_old = (T)st->rho[it0 & 1];
+    __syncthreads();
+    if (s_done) return;
+    const Waiter wt{&st->fault, a.wait_ticks, a.hm};
+    int lo = w.lo, hi = w.lo;
+    if (!SHARED) {                  // the columns this block reaches
+        lo = G > 1 && nloc > 0 ? halo_rows(rb - a.deps[2 * blk]) : 0;
+        hi = G > 1 && nloc > 0 ? halo_rows(a.deps[2 * blk + 1] + 1 - (rb + a.rows)) : 0;
+    }
+    const int alo = G > 1 ? a.deps[2 * blk] / a.rows : 0, ahi = G > 1 ? a.deps[2 * blk + 1] / a.rows : 0;
+    T* const lp = reinterpret_cast<T*>(res_lds);
+    T* const own = lp + lo;
+    for (size_t i = tid; i < w.lds / sizeof(T); i += kResThreads) lp[i] = T(0);   // read as a finite p (times 0) too
+    __syncthreads();
+    T xv[R], rv[R], sv[R], qv[R], u1[R], u2[R], dv[R];
+    RowSlots<T, SHARED> rows[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {   // past the block's rows: every vector 0, D = 1, no entries
+        const int l = k * kResThreads + tid;
+        xv[k] = rv[k] = sv[k] = qv[k] = u1[k] = u2[k] = T(0);
+        dv[k] = T(1);
+        if (l < nloc) {
+            xv[k] = a.x[rb + l];
+            rv[k] = a.r[rb + l];
+            sv[k] = shadow[rb + l];
+            dv[k] = a.D[rb + l];
+            if (it0 > 0) {
+                qv[k] = qg[rb + l];
+                u2[k] = u2g[rb + l];
+            }
+            if (a.keep) {           // the state a fallback starts from
+                a.keep[rb + l] = xv[k];
+                a.keep[(size_t)a.n + rb + l] = rv[k];
+            }
+        }
+        load_row(A, rb + l, l < nloc, w, rb - lo, lo + min(l, a.rows - 1), rows[k]);
+    }
+    constexpr int W = CoherentVec<T>::W;
+    const CoherentVec<T> zin(a.z, a.n);
+    const HaloRun below{0, rb - lo, lo / W}, above{lo + a.rows, rb + a.rows, hi / W};
+    uint32_t tag = a.tag;
+    int it = it0, niter = 0;
+    bool stop = false;
+    double err = 0.0;
+    for (;;) {
+        int t = tid;                // opaque, as in cg_window
+        asm volatile("" : "+v"(t));
+        // the product with the vector f(k) of row k: LDS, memory, halo, row sums into y
+        auto product = [&](auto&& f, auto&& y) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const int l = k * kResThreads + t;
+                const T p = f(k);
+                if (l < nloc) {
+                    own[l] = p;
+                    if (G > 1) coherent_store(a.z + rb + l, p);
+                }
+            }
+            if (G > 1) {
+                if (!neighbour_sync(a.flags, blk, alo, ahi, ++tag, wt, &s_fail)) return false;
+                halo_update<SHARED, R>(t, zin, lp, below, above, w, rb, a.rows, true, T(0));
+            }
+            __syncthreads();
+            int at = lo + t, off = 0;
+            asm volatile("" : "+v"(off));
+#pragma unroll
+            for (int k = 0; k < R; ++k) y(k, row_sum<SHARED, Op>(rows[k], k, at, off, w, lp));
+            return true;
+        };
+        T v[2] = {T(0), T(0)};
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            v[0] += rv[k] * rv[k];
+            v[1] += rv[k] * sv[k];                                  // rho, CGS.f90:118-122
+        }
+        if (!resident_sum<T, 2>(t, v, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
+        err = sqrt((double)v[0]);
+        if (err < tol) {
+            stop = true;
+            niter = it;
+            break;
+        }
+        if (it + 1 > cap) {
+            stop = true;
+            niter = (cap > 0 ? cap : 0) + 1;
+            break;
+        }
+        if (it - it0 == a.chunk) break;
+        const T rho = v[1];
+        const bool first = it == 0;
+        const T beta = first ? T(0) : rho / rho_old;
+        rho_old = rho;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            u1[k] = first ? rv[k] : rv[k] + beta * qv[k];
+            u2[k] = first ? rv[k] : u1[k] + beta * (qv[k] + beta * u2[k]);
+        }
+        T rs[1] = {T(0)};
+        if (!product([&](int k) { return u2[k] / dv[k]; },
+                     [&](int k, T y) {
+                         qv[k] = y;                                 // v, until alfa is known
+                         rs[0] += sv[k] * y;                        // (r2, v)  :215-219
+                     }))
+            return;
+        if (!resident_sum<T, 1>(t, rs, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
+        const T alfa = rho / rs[0];                                 // :220
+        if (!product(
+                [&](int k) {
+                    qv[k] = u1[k] - alfa * qv[k];                   // :226-228
+                    const T p = (u1[k] + qv[k]) / dv[k];            // :238-241
+                    xv[k] = xv[k] + alfa * p;                       // :286-288
+                    return p;
+                },
+                [&](int k, T y) { rv[k] = rv[k] - alfa * y; }))     // :315-317
+            return;
+        ++it;
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const int l = k * kResThreads + tid;
+        if (l < nloc) {
+            a.x[rb + l] = xv[k];
+            a.r[rb + l] = rv[k];
+            qg[rb + l] = qv[k];
+            u2g[rb + l] = u2[k];
+        }
+    }
+    if (lead) {
+        st->it = it;
+        st->rho[it & 1] = (double)rho_old;
+        st->error = err;
+        if (stop) {
+            st->done = 1;
+            st->niter_out = niter;
+        }
+    }
 }
 
 // Many systems in one launch: each has its own blocks, posts and state, and
@@ -987,8 +1157,6 @@ bool launch_cg_stream(const Op& A, const ResidentArgs<T>& a, int grid, hipStream
     if (R <= 6) return launch_resident(k_cg_stream<Op, 6>, grid, lds, s, A, a);
     return launch_resident(k_cg_stream<Op, 8>, grid, lds, s, A, a);
 }
-template bool launch_cg_stream<Sell<double>, double>(const Sell<double>&, const ResidentArgs<double>&, int,
-                                                     hipStream_t);
 template bool launch_cg_stream<Csr<double>, double>(const Csr<double>&, const ResidentArgs<double>&, int, hipStream_t);
 
 // the kernel of the fewest rows per thread that hold R (even ones, the FP32
@@ -1011,6 +1179,20 @@ bool launch_cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& 
     return A.soff ? launch_window<true>(std::integral_constant<int, 1>{}, R, A, a, w, grid, s)
                   : launch_window<false>(std::integral_constant<int, 1>{}, R, A, a, w, grid, s);
 }
+template <bool SHARED>
+static bool launch_cgs(int R, const Sell<double>& A, const ResidentArgs<double>& a, const WindowShape& w,
+                       const double* r2, double* q, double* u2, int grid, hipStream_t s) {
+    if (R <= 1) return launch_resident(k_cgs_window<Sell<double>, SHARED, 1>, grid, w.lds, s, A, a, w, r2, q, u2);
+    if (R <= 2) return launch_resident(k_cgs_window<Sell<double>, SHARED, 2>, grid, w.lds, s, A, a, w, r2, q, u2);
+    if (R <= kCgsRows) return launch_resident(k_cgs_window<Sell<double>, SHARED, 4>, grid, w.lds, s, A, a, w, r2, q, u2);
+    return false;
+}
+bool launch_cgs_window(const Sell<double>& A, const ResidentArgs<double>& a, const WindowShape& w, const double* r2,
+                       double* q, double* u2, int grid, hipStream_t s) {
+    const int R = (a.rows + kResThreads - 1) / kResThreads;
+    return A.soff ? launch_cgs<true>(R, A, a, w, r2, q, u2, grid, s) : launch_cgs<false>(R, A, a, w, r2, q, u2, grid, s);
+}
+
 template <int N>
 static bool launch_batch(std::integral_constant<int, N>, int R, int grid, size_t lds, const ResidentSystem* sys,
                          const int* blk_sys, uint32_t tag, hipStream_t s) {

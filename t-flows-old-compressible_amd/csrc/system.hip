@@ -1247,10 +1247,21 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     method = kernel_method(method);
     ws_.ensure((size_t)V_COUNT * n_);
     KrylovVectors<double> w = vectors(x, r1);
-    // CG on the chip where it fits (it reads no workspace that it or its
-    // set-up has not written)
-    const ResidentShape shape =
-        method == 0 && prec != 2 && cg_resident_enabled() ? resident_shape_of<double>() : ResidentShape{};
+    // CG and CGS on the chip where they fit (they read no workspace that they
+    // or their set-up have not written)
+    ResidentShape shape;
+    if (method != 1 && prec != 2 && cg_resident_enabled())
+        shape = method == 0 ? resident_shape_of<double>() : res_off_ ? ResidentShape{} : resident_shape(n_, kCgsRows);
+    ResidentSpace sp;
+    WindowShape win;
+    bool window = false;
+    if (shape.grid) {
+        sp = resident_space(shape, true, s);
+        // the rows in registers, unless their length or their columns' reach
+        // forbids it; CG, too, under TFLOWS_FP64_OP=csr, reads the CSR rows
+        window = (method == 2 || op64_env_ != 0) && window_of(shape, sell64(s), sell64_width_, sell64_offsets_, win);
+        if (method == 2 && !window) shape = ResidentShape{};
+    }
     // iteration 1 overwrites p, p2, u1, u2 before reading them; zero the
     // workspace anyway so no value of a previous solve lingers
     if (!shape.grid) TF_CHECK(hipMemsetAsync(ws_.p, 0, sizeof(double) * (size_t)V_COUNT * n_, s));
@@ -1271,23 +1282,18 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     bool resident = false;
     if (shape.grid) {
         start_solve<double, Csr<double>>(ctx(), method, prec, A, A, w, sites(), state_.p, mirror_, L, s, false, false);
-        launch_cgf_check(false, sites(), (const double*)nullptr, state_.p, mirror_, s);   // CG.f90:93-108
-        const ResidentSpace sp = resident_space(shape, true, s);
-        // the sliced operator, unless TFLOWS_FP64_OP=csr or rows of very
-        // uneven length pad it far
-        const bool csr_rows = op64_env_ == 0 || (sell64(s), sell64_entries_ > nnz_ + nnz_ / 2 + 64 * (int64_t)kSlice);
-        WindowShape win;
-        const bool window = !csr_rows && window_of(shape, sell64(s), sell64_width_, sell64_offsets_, win);
+        if (method == 0) launch_cgf_check(false, sites(), (const double*)nullptr, state_.p, mirror_, s);   // CG.f90:93-108
+        else launch_check(ctx(), 1, sites(), state_.p, mirror_, s);
         auto launch = [&](const ResidentArgs<double>& a) {
-            if (window) return launch_cg_window(sell64(s), a, win, shape.grid, s);
-            // (k_cg_stream reads columns, which a shared-offset copy does not hold)
-            return csr_rows || sell64(s).soff ? launch_cg_stream(A, a, shape.grid, s)
-                                              : launch_cg_stream(sell64(s), a, shape.grid, s);
+            if (method == 2) return launch_cgs_window(sell64(s), a, win, w.r2, w.q, w.u2, shape.grid, s);
+            return window ? launch_cg_window(sell64(s), a, win, shape.grid, s)
+                          : launch_cg_stream(A, a, shape.grid, s);
         };
         resident = run_resident(shape, sp, launch, w, state_.p, h, h2, s);
         if (!resident) {
             resident_gave_up();
-            launch_cgf_init_z(n_, (const double*)w.r1, (const double*)w.D, w.u1, sites(), state_.p, s);
+            if (method == 0)
+                launch_cgf_init_z(n_, (const double*)w.r1, (const double*)w.D, w.u1, sites(), state_.p, s);
         }
     }
     if (!resident) {

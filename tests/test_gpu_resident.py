@@ -132,6 +132,49 @@ def test_iterations_past_one_launch(pkg, cuda, monkeypatch, shape):
         assert np.linalg.norm(s.b - A @ x) <= s.tol + it * 2.2e-16 * norm_a * np.linalg.norm(x)
 
 
+@pytest.mark.parametrize("case", ["one_block", "last_block_short", "locality", "two_step", "locality_largest"])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_cgs_matches(pkg, oracle, cuda, monkeypatch, case, prec):
+    """CGS on the chip: 6 iterations against one launch per kernel (its
+    squared polynomial amplifies the rounding of the dot products; the
+    parity bar of a capped CGS is 1e-9), and the converged solve's true
+    residual."""
+    mg = pkg.meshgen
+    s = {"one_block": lambda: mg.momentum_system((15, 13, 11), seed=61, renumber=False),
+         "last_block_short": lambda: mg.momentum_system((19, 16, 17), seed=62),
+         "locality": lambda: mg.momentum_system((41, 37, 33), seed=63),
+         "two_step": lambda: mg.momentum_system((67, 53, 59), seed=64, renumber=False),
+         "locality_largest": lambda: mg.momentum_system((80, 80, 78), seed=65)}[case]()
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        out[mode] = (_solve(pkg, cuda, s, prec, 6, 0.0, "cgs"), _solve(pkg, cuda, s, prec, 600, s.tol, "cgs"))
+    (a, ac), (b, bc) = out["1"], out["0"]
+    assert a[0][0] == b[0][0] == 7 and a[0][1] == b[0][1]
+    assert _rel(a[1], b[1]) <= 1e-9
+    if s.matrix.n < 10000:
+        assert _rel(a[1], oracle.run("cgs", s.matrix, s.b, prec=prec, niter=6, tol=0.0)["x"]) <= 1e-9
+    if bc[0][0] <= 600:                # it converges without the on-chip form, too
+        # (the count is not compared: a CGS residual rises and falls by orders
+        # from one iteration to the next, so rounding decides which one first
+        # falls below tol; what its peaks lose, both forms lose alike)
+        A = s.matrix.to_scipy()
+        true = [np.linalg.norm(s.b - A @ v) for v in (ac[1], bc[1])]
+        assert ac[0][0] <= 600 and ac[0][2] < s.tol and true[0] < 10 * max(s.tol, true[1])
+
+
+def test_cgs_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
+    s = pkg.meshgen.momentum_system((40, 40, 41), seed=66, renumber=False)
+    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "0")
+    want = _solve(pkg, cuda, s, 1, 20, 0.0, "cgs")
+    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "1")
+    whole = _solve(pkg, cuda, s, 1, 20, 0.0, "cgs")
+    monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
+    got = _solve(pkg, cuda, s, 1, 20, 0.0, "cgs")
+    expect = want if "gave up waiting" in capfd.readouterr().err else whole
+    assert got[0] == expect[0] and np.array_equal(got[1], expect[1]) and np.array_equal(got[2], expect[2])
+
+
 def test_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
     """A synchronisation that waits beyond TFLOWS_BARRIER_WAIT_MS (0: at
     once) is given up by every block, and the solve runs one launch per
