@@ -8,10 +8,9 @@
 // Here:
 //   k_calcps_faces  one thread per face: SMDPN, the interpolated mass
 //                   velocities, A12 and the flux, in the reference's
-//                   operation order; writes the off-diagonal pair
-//                   Aval(SidAij(1:2,s)) = -A12, Abou, Flux(s) and the face's
-//                   diagonal term;
-//   k_calcps_cells  one thread per cell: the diagonal and b summed over the
+//                   operation order; writes Abou, Flux(s) and A12;
+//   k_calcps_cells  one thread per cell: the row's off-diagonals
+//                   Aval(SidAij(1:2,s)) = -A12; the diagonal and b summed over the
 //                   cell's faces in ascending face order -- the order in
 //                   which the reference's face loop reaches them, so both
 //                   are the reference's bit for bit (Nmat passes included);
@@ -71,9 +70,8 @@ __device__ __forceinline__ bool adds_diag(unsigned char k) {
     return k == kInterior || k == kBuffer || k == kDiagOut || k == kPressure;
 }
 
-__global__ __launch_bounds__(kBlock) void k_calcps_faces(CalcPSMesh M, CalcPSFields F, double* __restrict__ aval,
-                                                          double* __restrict__ flux, double* __restrict__ abou,
-                                                          double* __restrict__ fa12) {
+__global__ __launch_bounds__(kBlock) void k_calcps_faces(CalcPSMesh M, CalcPSFields F, double* __restrict__ flux,
+                                                          double* __restrict__ abou, double* __restrict__ fa12) {
     const int s = blockIdx.x * kBlock + threadIdx.x;
     if (s >= M.ns) return;
     const unsigned char k = M.kind[s];
@@ -113,12 +111,7 @@ __global__ __launch_bounds__(kBlock) void k_calcps_faces(CalcPSMesh M, CalcPSFie
     }
     // interior and BUFFER faces (:86-112)
     const double A12 = (0.5 * SMDPN) * (M.volume[nb + c1] / F.asave[nb + c1] + M.volume[nb + c2] / F.asave[nb + c2]);
-    if (k == kInterior) {
-        aval[M.sid1[s]] = -A12;
-        aval[M.sid2[s]] = -A12;
-    } else {
-        abou[nb + c2] = -A12;                                          // Abou(-NbC:-1)
-    }
+    if (k == kBuffer) abou[nb + c2] = -A12;                            // Abou(-NbC:-1)
     const double dPxi = (0.5 * (F.px[nb + c1] + F.px[nb + c2])) * Dx;
     const double dPyi = (0.5 * (F.py[nb + c1] + F.py[nb + c2])) * Dy;
     const double dPzi = (0.5 * (F.pz[nb + c1] + F.pz[nb + c2])) * Dz;
@@ -127,17 +120,26 @@ __global__ __launch_bounds__(kBlock) void k_calcps_faces(CalcPSMesh M, CalcPSFie
 }
 
 // Partials per block: max |b| before the time term, sum of b V, sum of V.
+// The thread of a cell also writes its row's off-diagonals, -A12 of the
+// face at SidAij(1,s) or SidAij(2,s) (:91-92): the face kernel wrote them
+// as 8-byte stores into rows that its x, y and z faces each reach at another
+// time (270 MB written for 132 at 1.25 M cells); here a row's entries, kept in
+// LDS until its loads are done, go out together.
+constexpr int kRowStaged = 6;   // off-diagonals per row staged in LDS (a hexahedron's faces)
 __global__ __launch_bounds__(kBlock) void k_calcps_cells(CalcPSMesh M, CalcPSFields F, int nmat, double dt,
                                                           const double* __restrict__ flux,
                                                           const double* __restrict__ fa12,
                                                           double* __restrict__ aval, double* __restrict__ b,
                                                           double* __restrict__ part) {
     const int nb = M.nbc;
+    __shared__ double st_val[kRowStaged][kBlock];
+    __shared__ int st_pos[kRowStaged][kBlock];
     double vmax = 0.0, sbv = 0.0, sv = 0.0;
     const int rb = blockIdx.x * kBlock + threadIdx.x;
     for (int i = rb; i < M.nc; i += gridDim.x * kBlock) {
         const int e0 = M.cptr[i], e1 = M.cptr[i + 1];
         double diag = 0.0, bb = 0.0;                                   // :51, :56
+        int staged = 0;
         for (int m = 0; m < nmat; ++m) {
             for (int e = e0; e < e1; ++e) {
                 const int code = M.cface[e];
@@ -145,10 +147,21 @@ __global__ __launch_bounds__(kBlock) void k_calcps_cells(CalcPSMesh M, CalcPSFie
                 const unsigned char k = M.kind[s];
                 if (k == kNone) continue;                              // no flux in the assembly
                 if (adds_diag(k)) diag = diag + fa12[s];
+                if (m == 0 && k == kInterior) {
+                    const int pos = (code & 1) ? M.sid2[s] : M.sid1[s];
+                    if (staged < kRowStaged) {
+                        st_val[staged][threadIdx.x] = -fa12[s];
+                        st_pos[staged][threadIdx.x] = pos;
+                        ++staged;
+                    } else {
+                        aval[pos] = -fa12[s];
+                    }
+                }
                 if (code & 1) bb = bb + flux[s];                       // the cell is c2
                 else bb = bb - flux[s];
             }
         }
+        for (int j = 0; j < staged; ++j) aval[st_pos[j][threadIdx.x]] = st_val[j][threadIdx.x];
         aval[M.adia[i]] = diag;
         vmax = fmax(vmax, fabs(bb));                                   // :173-175
         const int c = i + 1;
@@ -1050,8 +1063,8 @@ void CalcPS::assemble(int nmat, double dt, const CalcPSFields& F, double* aval, 
             hipLaunchKernelGGL(k_calcps_zero, dim3((n_zero_ + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n_zero_,
                                (const int*)zero_idx_, aval);
         if (ns_ > 0)
-            hipLaunchKernelGGL(k_calcps_faces, dim3((ns_ + kBlock - 1) / kBlock), dim3(kBlock), 0, s, M_, F, aval,
-                               flux, abou, fa12_);
+            hipLaunchKernelGGL(k_calcps_faces, dim3((ns_ + kBlock - 1) / kBlock), dim3(kBlock), 0, s, M_, F, flux,
+                               abou, fa12_);
     }
     hipLaunchKernelGGL(k_calcps_cells, dim3(grid_), dim3(kBlock), 0, s, M_, F, nmat, dt, (const double*)flux,
                        (const double*)fa12_, aval, b, part_);
