@@ -39,6 +39,15 @@
 // its next B before all have read the last C, and none posts C before all
 // have read the last B.
 //
+// Measured, us per iteration, one launch per kernel -> on the chip (FP64,
+// Jacobi): natural order 65,600 rows 12.9 -> 6.5, 230,580 17.0 -> 8.2,
+// 491,111 26.1 -> 9.1, 979,902 35.8 -> 12.6; locality order 230,580 rows
+// 18.2 -> 8.5, 506,880 28.9 -> 10.4; k_cg_stream (CSR rows) 65,600 rows
+// 14.8 -> 11.7, 491,111 28.5 -> 20.7, 979,902 40.8 -> 34.3.  At 491,111 rows
+// (256 blocks, 2.1 GHz) an iteration is 7400 cycles of synchronisation C,
+// 6100 of B, 3400 of halo, 1200 of row sums and 3000 of the rest: latency of
+// device-scope accesses, not bandwidth, bounds it.
+//
 // Every wait ends: the grid is at most one block per CU (the host checks
 // that the device holds it at once), and a wait longer than wait_ticks
 // (another process held the CUs) raises the fault word, on which every

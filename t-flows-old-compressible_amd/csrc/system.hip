@@ -1260,7 +1260,11 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
         // the rows in registers, unless their length or their columns' reach
         // forbids it; CG, too, under TFLOWS_FP64_OP=csr, reads the CSR rows
         window = (method == 2 || op64_env_ != 0) && window_of(shape, sell64(s), sell64_width_, sell64_offsets_, win);
-        if (method == 2 && !window) shape = ResidentShape{};
+        // CGS of a system of one block keeps the kernels: on small pressure
+        // matrices its count follows the reference loop's within one only
+        // with their summation by 256-row tiles (12^3: 134 iterations, 128 on
+        // the chip, from rounding alone)
+        if (method == 2 && (!window || shape.grid == 1)) shape = ResidentShape{};
     }
     // iteration 1 overwrites p, p2, u1, u2 before reading them; zero the
     // workspace anyway so no value of a previous solve lingers

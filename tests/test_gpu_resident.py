@@ -152,6 +152,8 @@ def test_cgs_matches(pkg, oracle, cuda, monkeypatch, case, prec):
     (a, ac), (b, bc) = out["1"], out["0"]
     assert a[0][0] == b[0][0] == 7 and a[0][1] == b[0][1]
     assert _rel(a[1], b[1]) <= 1e-9
+    if case == "one_block":            # keeps one launch per kernel
+        assert ac[0] == bc[0] and np.array_equal(ac[1], bc[1]) and np.array_equal(ac[2], bc[2])
     if s.matrix.n < 10000:
         assert _rel(a[1], oracle.run("cgs", s.matrix, s.b, prec=prec, niter=6, tol=0.0)["x"]) <= 1e-9
     if bc[0][0] <= 600:                # it converges without the on-chip form, too
