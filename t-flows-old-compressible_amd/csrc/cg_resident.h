@@ -4,13 +4,11 @@
 #include <vector>
 
 #include "krylov_kernels.h"
+#include "resident_window.h"
 
 namespace tflows {
 
-constexpr int kResThreads = 512;      // threads of a block
-constexpr size_t kResLdsBytes = 160 * 1024 - 16 * 1024;   // LDS of a CU less the kernel's own arrays
 constexpr int kResChunk = 1024;       // iterations of a launch: bounds how long it holds the CUs
-constexpr int kResMaxBlocks = 512;    // eight eighths of a wavefront's lanes
 constexpr int kPostWords = 4;         // 64-bit words a block posts at a site (two FP64 values)
 constexpr int kPostStride = kResMaxBlocks;            // words between two words of a block
 constexpr int kPostSite = kPostWords * kPostStride;   // words of a copy of a site's posts
@@ -22,58 +20,10 @@ constexpr int kPostTotal = 2 * kPostCopies * (kPostSite + kPostSecond);
 // replacement once it has dropped this far below the last FP64 norm
 constexpr double kReplaceDrop = 1e-2;
 
-// Blocks and rows of a block for n rows on the current device, at most
-// rows_per_thread x kResThreads rows in a block; grid 0 when the chip does
-// not hold them.
-struct ResidentShape {
-    int grid = 0, rows = 0;
-};
+// resident_shape on the current device
 ResidentShape resident_shape(int n, int rows_per_thread);
 // the most blocks of a launch: one per CU
 int resident_blocks();
-
-// rows of a thread that the registers hold: FP64 8 (14 of 256 registers per
-// row's values) and FP32 16 of a shared-offset matrix, half where every entry
-// also has its column (the locality order)
-template <typename T>
-constexpr int resident_rows_per_thread(bool reordered) {
-    return (sizeof(T) == 8 ? 8 : 16) / (reordered ? 2 : 1);
-}
-// the rows per thread of the kernel that runs R of them
-constexpr int window_kernel_rows(int R) { return R <= 1 ? R : R <= 8 ? (R + 1) / 2 * 2 : (R + 3) / 4 * 4; }
-// D in LDS, too, where a thread's rows would take too many registers
-template <typename T>
-constexpr bool window_d_in_lds(int kernel_rows) {
-    return kernel_rows * sizeof(T) >= 48;
-}
-// entries of a row k_cg_window keeps: those of a 7-point row, without the
-// diagonal in the FP32 difference form
-template <typename T>
-constexpr int window_slots() {
-    return sizeof(T) == 8 ? 7 : 6;
-}
-// rows of a halo of `need` rows: whole granules of 16 bytes
-__host__ __device__ constexpr int halo_rows(int need) { return need <= 0 ? 0 : (need + 3) / 4 * 4; }
-
-// LDS of k_cg_window.  The halo of a block of a shared-offset matrix: column
-// offsets shorter than a block lie within `lo` rows of the block; each longer
-// one (far) has a region of its own, as many rows as the block.
-constexpr int kMaxFar = 4;
-constexpr int kMaxWindowSlots = 7;
-struct WindowShape {
-    int lo = 0, nfar = 0, nslots = 0;
-    int farbase = 0;                          // LDS index of the first far region
-    int far[kMaxFar] = {};
-    int offset[kMaxWindowSlots] = {};         // the matrix's column offsets, ascending
-    int disp[kMaxWindowSlots] = {};           // LDS distance of each from the row's own p
-    size_t lds = 0;                           // bytes
-};
-// The shapes of a shared-offset matrix (its distinct column offsets) and of
-// any other (deps read back); false when the LDS does not hold them.
-template <typename T>
-bool window_shape(const ResidentShape& sh, const std::vector<int>& offsets, WindowShape& w);
-template <typename T>
-bool window_shape(const ResidentShape& sh, const std::vector<int>& deps, int n, WindowShape& w);
 
 template <typename T>
 struct ResidentArgs {

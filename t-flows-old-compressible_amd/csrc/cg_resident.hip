@@ -66,14 +66,6 @@ namespace tflows {
 namespace {
 
 constexpr int kResWaves = kResThreads / kWave;
-// one block up to this many rows: its synchronisations are block barriers
-constexpr int kResOneBlockRows = 4096;
-// else blocks of at least this many: below it the synchronisation of more
-// blocks costs more than the shorter row sums save; up to twice as many
-// where that keeps to the blocks that synchronise in one step (84,480 rows,
-// locality order: 64 blocks 11.6 ms, 80 blocks 13.9)
-constexpr int kResMinRows = 1024;
-
 __device__ __forceinline__ double coherent_load(const double* p) {
     const uint64_t u = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
@@ -236,6 +228,7 @@ __device__ __forceinline__ bool resident_sum(int tid, T (&v)[NV], uint64_t* slot
 // Synchronisation A: this block's published rows have reached memory, and
 // those of the blocks its columns reach (alo .. ahi) have.  False when the
 // wait was given up (the whole block agrees).
+static_assert(kResMaxBlocks <= kResThreads, "a thread for each block waited for");
 __device__ __forceinline__ bool neighbour_sync(uint32_t* flags, int blk, int alo, int ahi, uint32_t tag,
                                                const Waiter& wt, int* s_fail) {
     __builtin_amdgcn_s_waitcnt(0);
@@ -825,6 +818,10 @@ __global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T>
 //   B  (r2, v)                 -> alfa; q; w = (u1 + q) / D published
 //   A  -> halo, x += alfa w, r -= alfa A w
 //
+// A waits for every block whose rows the halo loads, those multiplied by 0
+// included (halo_reach): what they publish is finite, what the vector holds
+// before that need not be.
+//
 // qg, u2g carry q and u2 from launch to launch.
 template <typename Op, bool SHARED, int R, typename T = typename OpValue<Op>::type>
 __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T> a, WindowShape w,
@@ -853,7 +850,15 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
         lo = G > 1 && nloc > 0 ? halo_rows(rb - a.deps[2 * blk]) : 0;
         hi = G > 1 && nloc > 0 ? halo_rows(a.deps[2 * blk + 1] + 1 - (rb + a.rows)) : 0;
     }
-    const int alo = G > 1 ? a.deps[2 * blk] / a.rows : 0, ahi = G > 1 ? a.deps[2 * blk + 1] / a.rows : 0;
+    // the blocks whose rows the halo reads (neighbour_sync has a thread for
+    // each: at most kResMaxBlocks)
+    int alo = 0, ahi = 0;
+    if (G > 1) {
+        const RowRange reach =
+            halo_reach(w, SHARED, RowRange{a.deps[2 * blk], a.deps[2 * blk + 1]}, rb, a.rows, a.n);
+        alo = reach.first / a.rows;
+        ahi = reach.last / a.rows;
+    }
     T* const lp = reinterpret_cast<T*>(res_lds);
     T* const own = lp + lo;
     for (size_t i = tid; i < w.lds / sizeof(T); i += kResThreads) lp[i] = T(0);   // read as a finite p (times 0) too
@@ -1049,20 +1054,7 @@ int resident_blocks() {
 }
 
 ResidentShape resident_shape(int n, int rows_per_thread) {
-    ResidentShape r;
-    const int cus = resident_blocks();
-    if (n <= 0 || cus <= 0) return r;
-    int grid = 1;
-    if (n > kResOneBlockRows) {
-        grid = std::min(cus, (n + kResMinRows - 1) / kResMinRows);
-        if (grid > kWave && n <= kWave * 2 * kResMinRows) grid = kWave;
-        if (grid >= kNumXcd) grid = grid / kNumXcd * kNumXcd;
-    }
-    const int64_t rows = (((int64_t)n + grid - 1) / grid + kSlice - 1) / kSlice * kSlice;
-    if (rows > (int64_t)rows_per_thread * kResThreads) return r;
-    r.grid = grid;
-    r.rows = (int)rows;
-    return r;
+    return resident_shape(n, rows_per_thread, resident_blocks());
 }
 
 namespace {
@@ -1113,49 +1105,6 @@ static bool launch_resident(K kernel, int grid, size_t lds, hipStream_t s, const
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kResThreads), lds, s, args...);
     return true;
 }
-
-// values of LDS: own rows and halo (the reads of the threads past the
-// block's rows stay inside), and D
-template <typename T>
-static size_t window_elems(const ResidentShape& sh, int lo, int hi, int nfar) {
-    const int R = window_kernel_rows((sh.rows + kResThreads - 1) / kResThreads);
-    return (size_t)lo + hi + (size_t)nfar * sh.rows + (size_t)R * kResThreads * (window_d_in_lds<T>(R) ? 2 : 1);
-}
-
-template <typename T>
-bool window_shape(const ResidentShape& sh, const std::vector<int>& offsets, WindowShape& w) {
-    w = WindowShape{};
-    if ((int)offsets.size() > window_slots<T>()) return false;
-    for (int d : offsets) {
-        const int64_t ad = d < 0 ? -(int64_t)d : d;
-        if (ad < sh.rows) w.lo = std::max(w.lo, halo_rows((int)ad));
-        else if (w.nfar < kMaxFar) w.far[w.nfar++] = d;
-        else return false;
-    }
-    w.farbase = 2 * w.lo + sh.rows;
-    for (int d : offsets) {
-        w.disp[w.nslots] = d;
-        for (int f = 0; f < w.nfar; ++f)
-            if (w.far[f] == d) w.disp[w.nslots] = w.farbase + f * sh.rows - w.lo;
-        w.offset[w.nslots++] = d;
-    }
-    w.lds = sizeof(T) * window_elems<T>(sh, w.lo, w.lo, w.nfar);
-    return w.lds <= kResLdsBytes;
-}
-template <typename T>
-bool window_shape(const ResidentShape& sh, const std::vector<int>& deps, int n, WindowShape& w) {
-    w = WindowShape{};
-    size_t most = window_elems<T>(sh, 0, 0, 0);
-    for (int b = 0; b < sh.grid && sh.grid > 1 && (int64_t)b * sh.rows < n; ++b)
-        most = std::max(most, window_elems<T>(sh, halo_rows(b * sh.rows - deps[2 * b]),
-                                              halo_rows(deps[2 * b + 1] + 1 - (b + 1) * sh.rows), 0));
-    w.lds = sizeof(T) * most;
-    return w.lds <= kResLdsBytes;
-}
-template bool window_shape<double>(const ResidentShape&, const std::vector<int>&, WindowShape&);
-template bool window_shape<float>(const ResidentShape&, const std::vector<int>&, WindowShape&);
-template bool window_shape<double>(const ResidentShape&, const std::vector<int>&, int, WindowShape&);
-template bool window_shape<float>(const ResidentShape&, const std::vector<int>&, int, WindowShape&);
 
 template <typename Op, typename T>
 bool launch_cg_stream(const Op& A, const ResidentArgs<T>& a, int grid, hipStream_t s) {

@@ -165,6 +165,43 @@ def test_cgs_matches(pkg, oracle, cuda, monkeypatch, case, prec):
         assert ac[0][0] <= 600 and ac[0][2] < s.tol and true[0] < 10 * max(s.tol, true[1])
 
 
+@pytest.mark.parametrize("boxes", [[(16, 16, 16)] * 8, [(40, 40, 41)] * 2, [(70, 60, 25)] * 3, [(40, 40, 41)]])
+def test_cgs_of_boxes_numbered_one_after_another(pkg, cuda, monkeypatch, boxes):
+    """A block's halo is loaded whole: rows of a zone's last plane lack the
+    entry whose rows are loaded, and so do the empty blocks at the end, so it
+    goes beyond the blocks that the columns reach and has to wait for those,
+    too (tests/resident_window_check.cpp shows which).  What a solve that
+    ended in NaN has left in the workspace must not enter the next one."""
+    import scipy.sparse as sp
+    import torch
+    mg = pkg.meshgen
+    parts = [mg.momentum_system(b, seed=70 + q, renumber=False) for q, b in enumerate(boxes)]
+    A = mg.from_scipy(sp.block_diag([q.matrix.to_scipy() for q in parts], format="csr"))
+    b = np.concatenate([q.b for q in parts])
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        ds = pkg.krylov.DeviceSystem(A)
+        assert ds.fp64_layout()["shared"]
+        got = []
+        for _ in range(3):
+            x = torch.zeros(A.n, dtype=torch.float64, device=cuda)
+            r = torch.full((A.n,), float("nan"), dtype=torch.float64, device=cuda)
+            ds.solve("cgs", 1, x, r, 2, 0.0)
+            assert torch.isnan(x).all()
+            x.zero_()
+            r.copy_(torch.from_numpy(b))
+            res = ds.solve("cgs", 1, x, r, 6, 0.0)
+            got.append((res, x.cpu().numpy(), r.cpu().numpy()))
+        ds.close()
+        for g in got[1:]:
+            assert g[0] == got[0][0] and np.array_equal(g[1], got[0][1]) and np.array_equal(g[2], got[0][2])
+        out[mode] = got[0]
+    a, k = out["1"], out["0"]
+    assert a[0][0] == k[0][0] == 7 and np.isfinite(a[1]).all()
+    assert _rel(a[1], k[1]) <= 1e-9
+
+
 def test_cgs_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
     s = pkg.meshgen.momentum_system((40, 40, 41), seed=66, renumber=False)
     monkeypatch.setenv("TFLOWS_CG_RESIDENT", "0")
