@@ -68,8 +68,12 @@ inline uint32_t resident_tags(int chunk) { return 4u * (uint32_t)chunk + 4u; }
 // TFLOWS_CG_RESIDENT=0, or an explicit kernel-per-phase form (TFLOWS_CG_FORM,
 // TFLOWS_CG_CARRY), turns the on-chip CG off (read at every solve)
 bool cg_resident_enabled();
-// longest wait of a synchronisation in wall-clock ticks (TFLOWS_BARRIER_WAIT_MS)
+// longest wait of a synchronisation in wall-clock ticks
+// (TFLOWS_BARRIER_WAIT_MS; 0: a poll that finds a post missing gives up)
 uint64_t resident_wait_ticks();
+// TFLOWS_BARRIER_WAIT_MS below 0: a solve's first launch starts with its
+// fault word raised, as for a block that starts after another gave up
+bool resident_starts_given_up();
 
 // Launches whose blocks wait for each other need the CUs of all their blocks
 // at once.  Two of them started from two host threads could each hold a part

@@ -125,7 +125,7 @@ struct Waiter {
     HostMirror* hm;                 // told, too, so that a host that paces itself on it stops
     // false when the wait must be given up
     __device__ __forceinline__ bool keep_waiting(unsigned& polls, uint64_t& t0) const {
-        if ((++polls & 127u) != 0) return true;
+        if ((++polls & 127u) != 0 && ticks != 0) return true;
         const uint64_t now = (uint64_t)wall_clock64();
         if (polls == 128u) t0 = now;
         if (now - t0 > ticks || __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
@@ -639,7 +639,10 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
     const int tid = threadIdx.x;
     if (tid == 0) {
         s_fail = 0;
-        s_done = st->done | st->suspend | st->fault;
+        // a launch that keeps the state a fallback starts from keeps all of
+        // it: a block that starts after another has given up does so, too,
+        // and gives up at its first long wait
+        s_done = st->done | st->suspend | (a.keep ? 0 : st->fault);
     }
     const int rb = min(blk * a.rows, a.n), nloc = min(a.n - rb, a.rows);
     const bool lead = blk == 0 && tid == 0;
@@ -834,7 +837,7 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
     const int tid = threadIdx.x;
     if (tid == 0) {
         s_fail = 0;
-        s_done = st->done | st->fault;
+        s_done = st->done | (a.keep ? 0 : st->fault);   // as in cg_window
     }
     const int G = gridDim.x, blk = logical_block();
     const int rb = min(blk * a.rows, a.n), nloc = min(a.n - rb, a.rows);
@@ -1038,9 +1041,13 @@ static int device_cus() {
     return cus;
 }
 
-uint64_t resident_wait_ticks() {
+static long wait_ms_from_env() {
     const char* e = std::getenv("TFLOWS_BARRIER_WAIT_MS");
-    const long ms = e ? std::atol(e) : 2000;
+    return e ? std::atol(e) : 2000;
+}
+bool resident_starts_given_up() { return wait_ms_from_env() < 0; }
+uint64_t resident_wait_ticks() {
+    const long ms = wait_ms_from_env();
     int dev = 0, khz = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)

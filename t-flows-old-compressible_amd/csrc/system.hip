@@ -1204,6 +1204,7 @@ bool System::run_resident(const ResidentShape& shape, const ResidentSpace& sp,
     a.wait_ticks = resident_wait_ticks();
     a.st = st;
     a.keep = sp.keep;
+    if (resident_starts_given_up()) launch_set_int(&st->fault, 1, s);
     for (;;) {
         a.tag = *sp.tag;
         *sp.tag += resident_tags(a.chunk);

@@ -229,6 +229,42 @@ def test_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
     assert got[0] == expect[0] and np.array_equal(got[1], expect[1]) and np.array_equal(got[2], expect[2])
 
 
+@pytest.mark.parametrize("case", ["natural", "one_block", "locality", "csr_rows", "cgs", "cgs_locality"])
+def test_fallback_restores_every_row(pkg, cuda, monkeypatch, capfd, case):
+    """Blocks that start after another has given up (a bound below 0 raises
+    the fault word before the launch) still save their x and r, so that the
+    fallback starts from the inputs and not from an earlier solve's."""
+    import torch
+    mg = pkg.meshgen
+    method = "cgs" if case.startswith("cgs") else "cg"
+    s = {"natural": lambda: mg.pressure_system((40, 40, 41), seed=11),
+         "one_block": lambda: mg.pressure_system((16, 16, 16), seed=11),
+         "locality": lambda: mg.pressure_system((41, 37, 33), seed=6, perm_seed=2),
+         "csr_rows": lambda: mg.pressure_system((40, 40, 41), seed=11),
+         "cgs": lambda: mg.momentum_system((40, 40, 41), seed=66, renumber=False),
+         "cgs_locality": lambda: mg.momentum_system((41, 37, 33), seed=63)}[case]()
+    if case == "csr_rows":
+        monkeypatch.setenv("TFLOWS_FP64_OP", "csr")
+    rng = np.random.default_rng(5)
+    starts = [rng.standard_normal(s.matrix.n) for _ in range(2)]
+    rhs = [s.b, s.b + rng.standard_normal(s.matrix.n) * np.abs(s.b).max()]
+    out = {}
+    for mode in ("0", "1"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        monkeypatch.delenv("TFLOWS_BARRIER_WAIT_MS", raising=False)
+        ds = pkg.krylov.DeviceSystem(s.matrix)
+        for q in range(2):
+            x, r = torch.from_numpy(starts[q]).to(cuda), torch.from_numpy(rhs[q]).to(cuda)
+            res = ds.solve(method, 1, x, r, 6, 0.0)
+            torch.cuda.synchronize()
+            monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "-1")
+        ds.close()
+        out[mode] = (res, x.cpu().numpy(), r.cpu().numpy())
+        assert ("gave up waiting" in capfd.readouterr().err) == (mode == "1")
+    a, k = out["1"], out["0"]
+    assert a[0] == k[0] and np.array_equal(a[1], k[1]) and np.array_equal(a[2], k[2])
+
+
 def test_two_threads(pkg, cuda):
     """Solves from two host threads on their own streams, each a launch that
     needs many CUs at once, give what they give alone."""
