@@ -320,6 +320,31 @@ def test_mixed_matches(pkg, cuda, monkeypatch, shape):
     assert np.linalg.norm(A @ (a[1] - b[1])) <= 2 * s.tol
 
 
+def test_mixed_error_against_64_bits(pkg, cuda, monkeypatch):
+    """Capped mixed solves against FP64 CG of the same cap.  Both forms round
+    the same FP32 vectors and the on-chip one sums them in FP64, so its mean
+    error is no larger; single solves scatter (a factor of 1.8 either way, so
+    the mean of 16 by about 15 %, and 1.25 is the ratio's bar)."""
+    import torch
+    mg = pkg.meshgen
+    mean = {"1": 0.0, "0": 0.0}
+    for q, shape in enumerate([(64, 64, 64), (83, 61, 47), (70, 72, 51), (96, 64, 32)] * 4):
+        s = mg.pressure_system(shape, seed=80 + q)
+        ds = pkg.krylov.DeviceSystem(s.matrix)
+        b = torch.from_numpy(s.b.copy()).to(cuda)
+        want, r = torch.zeros_like(b), b.clone()
+        ds.solve("cg", 1, want, r, 220, 0.0)
+        for mode in mean:
+            monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+            x = torch.zeros_like(b)
+            ds.solve_mixed_reliable(1, x, b, 220, 0.0, interval=50)
+            mean[mode] += float((x - want).norm() / want.norm()) / 16
+        monkeypatch.delenv("TFLOWS_CG_RESIDENT")
+        ds.close()
+    print(f"mean error on the chip {mean['1']:.2e}, one launch per kernel {mean['0']:.2e}", flush=True)
+    assert mean["1"] <= 1.25 * mean["0"]
+
+
 def _batch(pkg, cuda, systems, form, caps, tols, prec=1, b=None):
     import torch
     B = pkg.krylov.DeviceBatch([s.matrix for s in systems])
