@@ -709,6 +709,7 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
             ra.tag = *sp.tag;
             *sp.tag += resident_tags(interval);
             resident = launch_cg_window(A32, ra, win, shape.grid, s);
+            if (!resident) resident_off(true);
         }
         if (!resident) with_op32(s, iterations);
         issued += interval;
@@ -736,7 +737,7 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
     (void)hipEventDestroy(ev[1]);
     if (h2.fault) {      // a launch gave up waiting: from the initial x again, one launch per kernel
         share.reset();
-        resident_gave_up();
+        resident_off(false);
         TF_CHECK(hipMemcpyAsync(x, sp.keep, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
         return solve_mixed_reliable_impl(prec, x, b, r_out, cap, tol, interval, outer_steps, s);
     }

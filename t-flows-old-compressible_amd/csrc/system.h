@@ -398,7 +398,8 @@ class System {
     // The iterations of a started Jacobi CG solve on the chip, to their end
     // (h: the state read back); launch(args) starts one launch.  False when a
     // wait was given up or the device does not hold the grid: x, r1 and the
-    // state are as before the first iteration again.
+    // state are as before the first iteration again, and the system keeps
+    // the kernel-per-phase form.
     bool run_resident(const ResidentShape& shape, const ResidentSpace& sp,
                       const std::function<bool(const ResidentArgs<double>&)>& launch, const KrylovVectors<double>& w,
                       SolverState* st, const SolverState& h0, SolverState& h, hipStream_t s);
@@ -409,7 +410,7 @@ class System {
     }
 
    private:
-    void resident_gave_up();
+    void resident_off(bool refused);
     ResidentSpace resident_space(const ResidentShape& shape, bool keep, hipStream_t s);
     // halo of k_cg_window for a sliced operator; false: the rows are too
     // long or the LDS too small

@@ -1146,10 +1146,13 @@ SolveResult System::solve_ext(int method, int prec, double* x, double* r1, int c
     return res;
 }
 
-void System::resident_gave_up() {
+// The system runs the kernel-per-phase form from now on.
+void System::resident_off(bool refused) {
     res_off_ = true;
-    std::fprintf(stderr, "libtflows_krylov: an on-chip CG launch gave up waiting (TFLOWS_BARRIER_WAIT_MS); this "
-                         "system now runs one launch per kernel\n");
+    std::fprintf(stderr, refused ? "libtflows_krylov: the device does not hold an on-chip launch at once; this system "
+                                   "now runs one launch per kernel\n"
+                                 : "libtflows_krylov: an on-chip CG launch gave up waiting (TFLOWS_BARRIER_WAIT_MS); "
+                                   "this system now runs one launch per kernel\n");
     std::fflush(stderr);
 }
 
@@ -1208,7 +1211,10 @@ bool System::run_resident(const ResidentShape& shape, const ResidentSpace& sp,
     for (;;) {
         a.tag = *sp.tag;
         *sp.tag += resident_tags(a.chunk);
-        if (!launch(a)) return false;
+        if (!launch(a)) {
+            resident_off(true);
+            return false;
+        }
         TF_CHECK(hipGetLastError());
         TF_CHECK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
         TF_CHECK(hipStreamSynchronize(s));
@@ -1220,6 +1226,7 @@ bool System::run_resident(const ResidentShape& shape, const ResidentSpace& sp,
     TF_CHECK(hipMemcpyAsync(w.r1, sp.keep + n_, sizeof(double) * n_, hipMemcpyDeviceToDevice, s));
     TF_CHECK(hipMemcpyAsync(st, &h0, sizeof(h0), hipMemcpyHostToDevice, s));
     TF_CHECK(hipStreamSynchronize(s));
+    resident_off(false);
     return false;
 }
 
@@ -1295,11 +1302,8 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
                           : launch_cg_stream(A, a, shape.grid, s);
         };
         resident = run_resident(shape, sp, launch, w, state_.p, h, h2, s);
-        if (!resident) {
-            resident_gave_up();
-            if (method == 0)
-                launch_cgf_init_z(n_, (const double*)w.r1, (const double*)w.D, w.u1, sites(), state_.p, s);
-        }
+        if (!resident && method == 0)
+            launch_cgf_init_z(n_, (const double*)w.r1, (const double*)w.D, w.u1, sites(), state_.p, s);
     }
     if (!resident) {
         with_op64(s, [&](const auto& Aop) {

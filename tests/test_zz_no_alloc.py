@@ -64,6 +64,29 @@ def test_noalloc_matches_solve(pkg, cuda, method, prec):
         ds.close()
 
 
+@pytest.mark.parametrize("wait", ["0", "-1"])
+def test_noalloc_fallback_is_kept(pkg, cuda, monkeypatch, capfd, wait):
+    """An on-chip launch that gives up (at its first poll, or started given
+    up) runs again, one launch per kernel, to that form's bits, and the
+    system keeps that form: the next calls launch nothing on the chip."""
+    s = pkg.meshgen.pressure_system(40, seed=81)
+    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "0")
+    ds = pkg.krylov.DeviceSystem(s.matrix)
+    want = _solve(pkg, ds, "tflows_solve", "cg", 1, s.b, 30, 0.0, cuda)
+    ds.close()
+    monkeypatch.delenv("TFLOWS_CG_RESIDENT")
+    ds = pkg.krylov.DeviceSystem(s.matrix)
+    monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", wait)
+    _same(_solve(pkg, ds, "tflows_solve_noalloc", "cg", 1, s.b, 30, 0.0, cuda), want)
+    assert capfd.readouterr().err.count("gave up waiting") == 1
+    _same(_solve(pkg, ds, "tflows_solve_noalloc", "cg", 1, s.b, 30, 0.0, cuda), want)
+    monkeypatch.delenv("TFLOWS_BARRIER_WAIT_MS")
+    for entry in ("tflows_solve_noalloc", "tflows_solve"):
+        _same(_solve(pkg, ds, entry, "cg", 1, s.b, 30, 0.0, cuda), want)
+    assert "gave up" not in capfd.readouterr().err
+    ds.close()
+
+
 def test_noalloc_refusals(pkg, cuda):
     mg = pkg.meshgen
     s = mg.pressure_system(10, seed=83)
