@@ -202,31 +202,46 @@ def test_cgs_of_boxes_numbered_one_after_another(pkg, cuda, monkeypatch, boxes):
     assert _rel(a[1], k[1]) <= 1e-9
 
 
-def test_cgs_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
-    s = pkg.meshgen.momentum_system((40, 40, 41), seed=66, renumber=False)
+@pytest.mark.parametrize("method", ["cg", "cgs"])
+def test_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd, method):
+    """A synchronisation that waits beyond TFLOWS_BARRIER_WAIT_MS is given up
+    by every block, and the solve runs one launch per kernel from its inputs,
+    to that form's bits.  With 0 the first poll that finds a post missing
+    gives up: some block's does, as not all of several blocks post before any
+    of them polls."""
+    mg = pkg.meshgen
+    s = (mg.pressure_system((40, 40, 41), seed=11) if method == "cg"
+         else mg.momentum_system((40, 40, 41), seed=66, renumber=False))
     monkeypatch.setenv("TFLOWS_CG_RESIDENT", "0")
-    want = _solve(pkg, cuda, s, 1, 20, 0.0, "cgs")
+    want = _solve(pkg, cuda, s, 1, 40, 0.0, method)
     monkeypatch.setenv("TFLOWS_CG_RESIDENT", "1")
-    whole = _solve(pkg, cuda, s, 1, 20, 0.0, "cgs")
     monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
-    got = _solve(pkg, cuda, s, 1, 20, 0.0, "cgs")
-    expect = want if "gave up waiting" in capfd.readouterr().err else whole
-    assert got[0] == expect[0] and np.array_equal(got[1], expect[1]) and np.array_equal(got[2], expect[2])
+    got = _solve(pkg, cuda, s, 1, 40, 0.0, method)
+    assert capfd.readouterr().err.count("gave up waiting") == 1
+    assert got[0] == want[0] and np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
 
 
-def test_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
-    """A synchronisation that waits beyond TFLOWS_BARRIER_WAIT_MS (0: at
-    once) is given up by every block, and the solve runs one launch per
-    kernel from its inputs, to that form's bits."""
-    s = pkg.meshgen.pressure_system((40, 40, 41), seed=11)
-    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "0")
-    want = _solve(pkg, cuda, s, 1, 40, 0.0)
-    monkeypatch.setenv("TFLOWS_CG_RESIDENT", "1")
-    whole = _solve(pkg, cuda, s, 1, 40, 0.0)
-    monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
-    got = _solve(pkg, cuda, s, 1, 40, 0.0)
-    expect = want if "gave up waiting" in capfd.readouterr().err else whole
-    assert got[0] == expect[0] and np.array_equal(got[1], expect[1]) and np.array_equal(got[2], expect[2])
+def test_mixed_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
+    import torch
+    s = pkg.meshgen.pressure_system((40, 40, 41), seed=14)
+    b = torch.from_numpy(s.b.copy()).to(cuda)
+    out = {}
+    for mode, wait in (("0", "2000"), ("1", "0"), ("1", "2000")):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", wait)
+        ds = pkg.krylov.DeviceSystem(s.matrix)
+        for _ in range(2):             # the second call keeps the form
+            x = torch.from_numpy(np.random.default_rng(9).standard_normal(s.matrix.n)).to(cuda)
+            r = torch.zeros_like(x)
+            res = ds.solve_mixed_reliable(1, x, b, 120, 0.0, interval=40, r_out=r)
+            torch.cuda.synchronize()
+            out.setdefault((mode, wait), []).append((res, x.cpu().numpy(), r.cpu().numpy()))
+        ds.close()
+        assert capfd.readouterr().err.count("gave up waiting") == (wait == "0")
+    for g in out["1", "0"] + out["0", "2000"]:
+        w = out["0", "2000"][0]
+        assert g[0] == w[0] and np.array_equal(g[1], w[1]) and np.array_equal(g[2], w[2])
+    assert not np.array_equal(out["1", "2000"][0][1], out["0", "2000"][0][1])   # the on-chip form's own bits
 
 
 @pytest.mark.parametrize("case", ["natural", "one_block", "locality", "csr_rows", "cgs", "cgs_locality"])
@@ -408,7 +423,6 @@ def test_batch_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
     whole = _batch(pkg, cuda, systems, 0, caps, tols)[0]
     monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
     got = _batch(pkg, cuda, systems, 0, caps, tols)[0]
-    gave_up = "gave up waiting" in capfd.readouterr().err
+    assert capfd.readouterr().err.count("gave up waiting") == 1
     for q in range(2):
-        assert got[0]["niter"][q] == 31
-        assert _rel(got[1][q], whole[1][q]) <= 1e-11 if gave_up else np.array_equal(got[1][q], whole[1][q])
+        assert got[0]["niter"][q] == 31 and _rel(got[1][q], whole[1][q]) <= 1e-11
