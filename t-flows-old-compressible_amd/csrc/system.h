@@ -409,6 +409,18 @@ class System {
         return res_off_ ? ResidentShape{} : resident_shape(n_, resident_rows_per_thread<T>(reordered_));
     }
 
+    // the same for FP64 CG: mesh rows only.  A thread of k_cg_stream reads its
+    // row by itself, entry after entry, so long rows cost it more than the
+    // kernels, whose blocks read them together: on / off the chip, 60
+    // iterations, ms, rows of 7 with a few of 11 entries 0.87 / 0.99 (65,600
+    // rows) 1.57 / 1.88 (493,039) 2.53 / 2.54 (970,299); all of 9 entries
+    // 1.02 / 0.98 (100,000) 2.58 / 2.52 (900,000), of 27 4.67 / 2.05
+    // (216,000), of 199 92.7 / 3.6 (4,000).  k_cg_window's rows are shorter
+    // than either bound.
+    ResidentShape resident_cg_shape() const {
+        return max_row_ <= 12 && nnz_ <= 7.5 * n_ ? resident_shape_of<double>() : ResidentShape{};
+    }
+
    private:
     void resident_off(bool refused);
     ResidentSpace resident_space(const ResidentShape& shape, bool keep, hipStream_t s);

@@ -1259,7 +1259,7 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     // or their set-up have not written)
     ResidentShape shape;
     if (method != 1 && prec != 2 && cg_resident_enabled())
-        shape = method == 0 ? resident_shape_of<double>() : res_off_ ? ResidentShape{} : resident_shape(n_, kCgsRows);
+        shape = method == 0 ? resident_cg_shape() : res_off_ ? ResidentShape{} : resident_shape(n_, kCgsRows);
     ResidentSpace sp;
     WindowShape win;
     bool window = false;

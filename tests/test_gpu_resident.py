@@ -115,6 +115,61 @@ def test_shared_offsets_beyond_the_window(pkg, oracle, cuda, monkeypatch):
         assert _rel(out["1"][1], out["0"][1]) <= 1e-12 and _residuals_agree(s, out["1"], out["0"])
 
 
+def _graph(pkg, n, offsets, rows=None, seed=3):
+    """Symmetric diagonally dominant matrix: entries i, i + d for the offsets,
+    and for a few rows i, i + 2, i + 5, ... (`rows`: how many more)."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    A = sp.diags([rng.uniform(0.5, 1.0, n - d) for d in offsets], offsets, shape=(n, n), format="csr")
+    if rows:
+        r = np.repeat(rng.choice(n - 100, n // 20, replace=False), rows)
+        A = A + sp.csr_matrix((np.full(len(r), 0.01), (r, r + np.tile(2 + 3 * np.arange(rows), n // 20))), shape=(n, n))
+    A = A + A.T
+    A = (sp.diags(np.asarray(A.sum(axis=1)).ravel() * 1.01) - A).tocsr()
+    A.sort_indices()
+    m = pkg.meshgen.from_scipy(A)
+    return pkg.meshgen.LinearSystem(m, rng.standard_normal(n), np.zeros(n), 1e-8, 1, 100, {})
+
+
+@pytest.mark.parametrize("case", ["rows_9", "rows_27", "rows_199_one_block", "dense_row"])
+def test_long_rows_keep_the_kernels(pkg, cuda, monkeypatch, case):
+    """Rows longer than a mesh's run one launch per kernel either way: the
+    same bits (a thread of the on-chip form reads its row entry by entry,
+    which takes up to 25 times as long as the kernels on such rows)."""
+    import scipy.sparse as sp
+    if case == "dense_row":
+        A = _graph(pkg, 20000, [1, 50, 2500]).matrix.to_scipy().tolil()
+        A[10000, :4000] = -1e-3
+        A[:4000, 10000] = -1e-3
+        m = pkg.meshgen.from_scipy(sp.csr_matrix(A))
+        s = pkg.meshgen.LinearSystem(m, np.ones(m.n), np.zeros(m.n), 1e-8, 1, 100, {})
+    else:
+        s = {"rows_9": lambda: _graph(pkg, 20000, [1, 50, 2500, 2501]),
+             "rows_27": lambda: _graph(pkg, 20000, [1, 29, 30, 31, 869, 870, 871, 899, 900, 901, 929, 930, 931]),
+             "rows_199_one_block": lambda: _graph(pkg, 4000, list(range(1, 100)))}[case]()
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        out[mode] = _solve(pkg, cuda, s, 1, 12, 0.0)
+    a, b = out["1"], out["0"]
+    assert a[0] == b[0] and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("n", [3000, 20000, 90000])
+def test_rows_of_a_refined_mesh(pkg, cuda, monkeypatch, n):
+    """Rows of 7 with some of up to 12 entries: on the chip, their rows read
+    every iteration."""
+    s = _graph(pkg, n, [1, 40, 1600], rows=2)
+    assert 8 <= np.diff(s.matrix.to_scipy().indptr).max() <= 12
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        out[mode] = _solve(pkg, cuda, s, 1, 12, 0.0)
+    a, b = out["1"], out["0"]
+    assert a[0][0] == b[0][0] == 13 and _rel(a[1], b[1]) <= 1e-12 and _residuals_agree(s, a, b)
+    assert not np.array_equal(a[2], b[2])      # the on-chip form's own sums
+
+
 @pytest.mark.parametrize("shape", [(2500, 1, 1), (9000, 1, 1)])
 def test_iterations_past_one_launch(pkg, cuda, monkeypatch, shape):
     """A launch runs at most 1024 iterations; the next one goes on from its
