@@ -820,7 +820,7 @@ __global__ __launch_bounds__(kResThreads) void k_cg_window(Op A, ResidentArgs<T>
 // included (halo_reach): what they publish is finite, what the vector holds
 // before that need not be.
 //
-// qg, u2g carry q and u2 from launch to launch.
+// qg, u2g carry q and u2 from launch to launch.  The grid is two blocks or more.
 template <typename Op, bool SHARED, int R, typename T = typename OpValue<Op>::type>
 __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T> a, WindowShape w,
                                                             const T* __restrict__ shadow, T* __restrict__ qg,
@@ -845,18 +845,13 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
     const Waiter wt{&st->fault, a.wait_ticks, a.hm};
     int lo = w.lo, hi = w.lo;
     if (!SHARED) {                  // the columns this block reaches
-        lo = G > 1 && nloc > 0 ? halo_rows(rb - a.deps[2 * blk]) : 0;
-        hi = G > 1 && nloc > 0 ? halo_rows(a.deps[2 * blk + 1] + 1 - (rb + a.rows)) : 0;
+        lo = nloc > 0 ? halo_rows(rb - a.deps[2 * blk]) : 0;
+        hi = nloc > 0 ? halo_rows(a.deps[2 * blk + 1] + 1 - (rb + a.rows)) : 0;
     }
     // the blocks whose rows the halo reads (neighbour_sync has a thread for
     // each: at most kResMaxBlocks)
-    int alo = 0, ahi = 0;
-    if (G > 1) {
-        const RowRange reach =
-            halo_reach(w, SHARED, RowRange{a.deps[2 * blk], a.deps[2 * blk + 1]}, rb, a.rows, a.n);
-        alo = reach.first / a.rows;
-        ahi = reach.last / a.rows;
-    }
+    const RowRange reach = halo_reach(w, SHARED, RowRange{a.deps[2 * blk], a.deps[2 * blk + 1]}, rb, a.rows, a.n);
+    const int alo = reach.first / a.rows, ahi = reach.last / a.rows;
     T* const lp = reinterpret_cast<T*>(res_lds);
     T* const own = lp + lo;
     for (size_t i = tid; i < w.lds / sizeof(T); i += kResThreads) lp[i] = T(0);   // read as a finite p (times 0) too
@@ -902,13 +897,11 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
                 const T p = f(k);
                 if (l < nloc) {
                     own[l] = p;
-                    if (G > 1) coherent_store(a.z + rb + l, p);
+                    coherent_store(a.z + rb + l, p);
                 }
             }
-            if (G > 1) {
-                if (!neighbour_sync(a.flags, blk, alo, ahi, ++tag, wt, &s_fail)) return false;
-                halo_update<SHARED, R>(t, zin, lp, below, above, w, rb, a.rows, true, T(0));
-            }
+            if (!neighbour_sync(a.flags, blk, alo, ahi, ++tag, wt, &s_fail)) return false;
+            halo_update<SHARED, R>(t, zin, lp, below, above, w, rb, a.rows, true, T(0));
             __syncthreads();
             int at = lo + t, off = 0;
             asm volatile("" : "+v"(off));
@@ -1142,7 +1135,6 @@ bool launch_cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& 
 template <bool SHARED>
 static bool launch_cgs(int R, const Sell<double>& A, const ResidentArgs<double>& a, const WindowShape& w,
                        const double* r2, double* q, double* u2, int grid, hipStream_t s) {
-    if (R <= 1) return launch_resident(k_cgs_window<Sell<double>, SHARED, 1>, grid, w.lds, s, A, a, w, r2, q, u2);
     if (R <= 2) return launch_resident(k_cgs_window<Sell<double>, SHARED, 2>, grid, w.lds, s, A, a, w, r2, q, u2);
     if (R <= kCgsRows) return launch_resident(k_cgs_window<Sell<double>, SHARED, 4>, grid, w.lds, s, A, a, w, r2, q, u2);
     return false;

@@ -637,14 +637,12 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
     // CSR: the same bits)
     // The FP32 iterations between two replacements on the chip where they
     // fit: one launch of cg_resident.hip each
-    const ResidentShape shape =
-        cg_resident_enabled() && interval <= 4 * kResChunk ? resident_shape_of<float>() : ResidentShape{};
+    const ResidentShape shape = interval <= 4 * kResChunk ? resident_shape_of<float>() : ResidentShape{};
     ResidentSpace sp;
-    WindowShape win;
     bool resident = false;
     if (shape.grid) {
         sp = resident_space(shape, true, s);
-        resident = window_of(shape, sell32(s), sell_width_, sell_offsets_, win);
+        resident = window32(shape, s);
     }
     const DiffSell32 A32 = resident ? sell32(s) : DiffSell32{};
     std::unique_ptr<CuShare> share;
@@ -708,7 +706,7 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
         if (resident) {
             ra.tag = *sp.tag;
             *sp.tag += resident_tags(interval);
-            resident = launch_cg_window(A32, ra, win, shape.grid, s);
+            resident = launch_cg_window(A32, ra, win32_, shape.grid, s);
             if (!resident) resident_off(true);
         }
         if (!resident) with_op32(s, iterations);

@@ -139,7 +139,7 @@ SolveResult solve_noalloc(System& S, int method, int prec, double* x, double* r1
     // on the chip, as System::solve does, where it fits
     SolverState h;
     bool resident = false;
-    const ResidentShape shape = cg_resident_enabled() ? S.resident_cg_shape() : ResidentShape{};
+    const ResidentShape shape = S.resident_cg_shape();
     if (shape.grid) {
         SolverState h0{};
         h0.tol = tol;

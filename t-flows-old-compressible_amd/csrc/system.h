@@ -139,7 +139,8 @@ bool slot_offsets16(int n, const std::vector<int>& off, const std::vector<int>& 
 bool col16_from_env(const char* name);
 void slice_layout(int n, const std::vector<int>& rp, const std::vector<int>& cl, bool pad_own, std::vector<int>& off,
                   std::vector<int>& col, std::vector<int>& map);
-// the distinct column offsets and the most slots of a slice of a sliced layout
+// the distinct column offsets (ascending; more than kMaxWindowSlots: some of
+// them) and the most slots of a slice of a sliced layout
 void slot_summary(const std::vector<int>& off, const std::vector<int>& soff, std::vector<int>& offsets, int& width);
 bool shared_slots_from_env();
 
@@ -403,12 +404,12 @@ class System {
     bool run_resident(const ResidentShape& shape, const ResidentSpace& sp,
                       const std::function<bool(const ResidentArgs<double>&)>& launch, const KrylovVectors<double>& w,
                       SolverState* st, const SolverState& h0, SolverState& h, hipStream_t s);
-    // blocks and rows of the on-chip CG (grid 0: not this system)
+    // blocks and rows of the on-chip forms (grid 0: not this system)
     template <typename T>
     ResidentShape resident_shape_of() const {
-        return res_off_ ? ResidentShape{} : resident_shape(n_, resident_rows_per_thread<T>(reordered_));
+        return res_off_ || !cg_resident_enabled() ? ResidentShape{}
+                                                  : resident_shape(n_, resident_rows_per_thread<T>(reordered_));
     }
-
     // the same for FP64 CG: mesh rows only.  A thread of k_cg_stream reads its
     // row by itself, entry after entry, so long rows cost it more than the
     // kernels, whose blocks read them together: on / off the chip, 60
@@ -424,10 +425,12 @@ class System {
    private:
     void resident_off(bool refused);
     ResidentSpace resident_space(const ResidentShape& shape, bool keep, hipStream_t s);
-    // halo of k_cg_window for a sliced operator; false: the rows are too
-    // long or the LDS too small
-    template <typename Op>
-    bool window_of(const ResidentShape& shape, const Op& A, int width, const std::vector<int>& offsets,
+    // whether k_cg_window holds the sliced operator (win64_, win32_: its
+    // LDS); not when the rows are too long or the LDS too small
+    bool window64(const ResidentShape& shape, hipStream_t s);
+    bool window32(const ResidentShape& shape, hipStream_t s);
+    template <typename T>
+    bool window_of(const ResidentShape& shape, bool shared, int width, const std::vector<int>& offsets,
                    WindowShape& w) const;
     SolveResult solve_ext(int method, int prec, double* x, double* r1, int cap, double tol, double stale_error,
                           hipStream_t s);
@@ -495,6 +498,8 @@ class System {
     std::vector<int> res_deps_h_;
     std::vector<int> sell64_offsets_, sell_offsets_;   // distinct column offsets of the shared-offset layouts
     int sell64_width_ = 0, sell_width_ = 0;            // most slots of a slice
+    int win64_fits_ = 2, win32_fits_ = 2;              // 2: not asked yet
+    WindowShape win64_, win32_;
     bool res_off_ = false;          // a wait was given up: kernel per phase from now on
     DevArray<float> off_val_, rowsum32_, diag32_;
     bool diff32_valid_ = false;

@@ -154,9 +154,11 @@ void slice_layout(int n, const std::vector<int>& rp, const std::vector<int>& cl,
 }
 
 void slot_summary(const std::vector<int>& off, const std::vector<int>& soff, std::vector<int>& offsets, int& width) {
-    offsets = soff;
-    std::sort(offsets.begin(), offsets.end());
-    offsets.erase(std::unique(offsets.begin(), offsets.end()), offsets.end());
+    offsets.clear();
+    for (size_t j = 0; j < soff.size() && (int)offsets.size() <= kMaxWindowSlots; ++j) {
+        const auto at = std::lower_bound(offsets.begin(), offsets.end(), soff[j]);
+        if (at == offsets.end() || *at != soff[j]) offsets.insert(at, soff[j]);
+    }
     width = 0;
     for (size_t sl = 0; sl + 1 < off.size(); ++sl) width = std::max(width, (off[sl + 1] - off[sl]) / kSlice);
 }
@@ -1230,18 +1232,36 @@ bool System::run_resident(const ResidentShape& shape, const ResidentSpace& sp,
     return false;
 }
 
-template <typename Op>
-bool System::window_of(const ResidentShape& shape, const Op& A, int width, const std::vector<int>& offsets,
-                       WindowShape& w) const {
-    using T = typename OpValue<Op>::type;
-    if (width > window_slots<T>()) return false;
-    if (!A.soff && shape.rows > resident_rows_per_thread<T>(true) * kResThreads) return false;
-    return A.soff ? window_shape<T>(shape, offsets, w) : window_shape<T>(shape, res_deps_h_, n_, w);
+// The pattern decides, so once per system (the values' form, full or
+// symmetric, has the same slots); an operator that is not used is not built
+// or filled again.
+bool System::window64(const ResidentShape& shape, hipStream_t s) {
+    if (win64_fits_ == 2) {
+        win64_fits_ = 0;
+        if (max_row_ <= window_slots<double>()) {
+            const Sell<double> A = sell64(s);
+            win64_fits_ = window_of<double>(shape, A.soff != nullptr, sell64_width_, sell64_offsets_, win64_);
+        }
+    }
+    return win64_fits_ == 1;
 }
-template bool System::window_of<Sell<double>>(const ResidentShape&, const Sell<double>&, int, const std::vector<int>&,
-                                              WindowShape&) const;
-template bool System::window_of<DiffSell32>(const ResidentShape&, const DiffSell32&, int, const std::vector<int>&,
-                                            WindowShape&) const;
+bool System::window32(const ResidentShape& shape, hipStream_t s) {
+    if (win32_fits_ == 2) {
+        win32_fits_ = 0;
+        if (max_row_ - 1 <= window_slots<float>()) {
+            const DiffSell32 A = sell32(s);
+            win32_fits_ = window_of<float>(shape, A.soff != nullptr, sell_width_, sell_offsets_, win32_);
+        }
+    }
+    return win32_fits_ == 1;
+}
+template <typename T>
+bool System::window_of(const ResidentShape& shape, bool shared, int width, const std::vector<int>& offsets,
+                       WindowShape& w) const {
+    if (width > window_slots<T>()) return false;
+    if (!shared && shape.rows > resident_rows_per_thread<T>(true) * kResThreads) return false;
+    return shared ? window_shape<T>(shape, offsets, w) : window_shape<T>(shape, res_deps_h_, n_, w);
+}
 
 int kernel_method(int method) {
     if (method != 1) return method;
@@ -1256,23 +1276,22 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     ws_.ensure((size_t)V_COUNT * n_);
     KrylovVectors<double> w = vectors(x, r1);
     // CG and CGS on the chip where they fit (they read no workspace that they
-    // or their set-up have not written)
+    // or their set-up have not written).  CGS of a system of one block keeps
+    // the kernels: on small pressure matrices its count follows the reference
+    // loop's within one only with their summation by 256-row tiles (12^3: 134
+    // iterations, 128 on the chip, from rounding alone)
     ResidentShape shape;
-    if (method != 1 && prec != 2 && cg_resident_enabled())
-        shape = method == 0 ? resident_cg_shape() : res_off_ ? ResidentShape{} : resident_shape(n_, kCgsRows);
+    if (method == 0 && prec != 2) shape = resident_cg_shape();
+    if (method == 2 && prec != 2 && !res_off_ && cg_resident_enabled()) shape = resident_shape(n_, kCgsRows);
+    if (method == 2 && shape.grid == 1) shape = ResidentShape{};
     ResidentSpace sp;
-    WindowShape win;
     bool window = false;
     if (shape.grid) {
         sp = resident_space(shape, true, s);
         // the rows in registers, unless their length or their columns' reach
         // forbids it; CG, too, under TFLOWS_FP64_OP=csr, reads the CSR rows
-        window = (method == 2 || op64_env_ != 0) && window_of(shape, sell64(s), sell64_width_, sell64_offsets_, win);
-        // CGS of a system of one block keeps the kernels: on small pressure
-        // matrices its count follows the reference loop's within one only
-        // with their summation by 256-row tiles (12^3: 134 iterations, 128 on
-        // the chip, from rounding alone)
-        if (method == 2 && (!window || shape.grid == 1)) shape = ResidentShape{};
+        window = (method == 2 || op64_env_ != 0) && window64(shape, s);
+        if (method == 2 && !window) shape = ResidentShape{};
     }
     // iteration 1 overwrites p, p2, u1, u2 before reading them; zero the
     // workspace anyway so no value of a previous solve lingers
@@ -1297,8 +1316,8 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
         if (method == 0) launch_cgf_check(false, sites(), (const double*)nullptr, state_.p, mirror_, s);   // CG.f90:93-108
         else launch_check(ctx(), 1, sites(), state_.p, mirror_, s);
         auto launch = [&](const ResidentArgs<double>& a) {
-            if (method == 2) return launch_cgs_window(sell64(s), a, win, w.r2, w.q, w.u2, shape.grid, s);
-            return window ? launch_cg_window(sell64(s), a, win, shape.grid, s)
+            if (method == 2) return launch_cgs_window(sell64(s), a, win64_, w.r2, w.q, w.u2, shape.grid, s);
+            return window ? launch_cg_window(sell64(s), a, win64_, shape.grid, s)
                           : launch_cg_stream(A, a, shape.grid, s);
         };
         resident = run_resident(shape, sp, launch, w, state_.p, h, h2, s);
