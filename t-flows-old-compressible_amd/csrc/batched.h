@@ -179,7 +179,7 @@ class Batch {
     bool persistent_ok_ = true;
     int resident_ = 2;                   // 2: not tried; 1: waves_ built; 0: kernel forms only
     std::vector<std::unique_ptr<ResidentWave>> waves_;
-    DevArray<uint64_t> res_posts_;       // kPostTotal words per system of several blocks
+    DevArray<uint64_t> res_posts_;       // kPostTotal words per system of several blocks of a launch
     uint32_t res_tag_ = 0;
     DevArray<int> bar_, pfault_;       // barrier counters (one per system) and the fault word of the persistent form
     uint64_t wait_ticks_ = 0;

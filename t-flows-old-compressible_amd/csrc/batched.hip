@@ -926,8 +926,14 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
     const BatchCtx c0 = ctx(1, false);
     start_solve<double, Csr<double>>(c0, 0, prec, A, A, w, S, st_.p, nullptr, &kNoLevels, bs_, false, false);
     launch_check(c0, 1, S, st_.p, nullptr, bs_);
-    const size_t words = (size_t)kPostTotal * k_;
-    if (!res_posts_.p || res_tag_ > (1u << 30)) {
+    // posts for the systems of several blocks, shared by the launches (they
+    // follow each other, and each numbers its synchronisations on)
+    int posters = 0;
+    for (const auto& wv : waves_)
+        posters = std::max(posters, (int)std::count_if(wv->sys.begin(), wv->sys.end(),
+                                                       [](const ResidentSystem& s) { return s.grid > 1; }));
+    if (posters && (!res_posts_.p || res_tag_ > (1u << 30))) {
+        const size_t words = (size_t)kPostTotal * posters;
         res_posts_.ensure(words);
         TF_CHECK(hipMemsetAsync(res_posts_.p, 0, sizeof(uint64_t) * words, bs_));
         res_tag_ = 0;
@@ -935,6 +941,7 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
     bool ok = true;
     out.resize(k_);
     for (auto& wv : waves_) {
+        int post = 0;
         for (size_t j = 0; j < wv->sys.size(); ++j) {
             ResidentSystem& s = wv->sys[j];
             const int q = wv->index[j], r0 = roff_[q];
@@ -945,8 +952,8 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
             s.a.p = w.p + r0;
             s.a.z = w.u1 + r0;
             s.a.D = w.D + r0;
-            s.a.slotB = res_posts_.p + (size_t)kPostTotal * q;
-            s.a.slotC = s.a.slotB + kPostTotal / 2;
+            s.a.slotB = s.grid > 1 ? res_posts_.p + (size_t)kPostTotal * post++ : nullptr;
+            s.a.slotC = s.grid > 1 ? s.a.slotB + kPostTotal / 2 : nullptr;
             s.a.wait_ticks = wait_ticks_;
             s.a.st = st_.p + q;
         }

@@ -471,6 +471,22 @@ def test_batch_of_several_launches(pkg, cuda):
         assert _rel(a[1][q], ref[1][q]) <= 1e-12
 
 
+def test_batch_of_small_systems_keeps_its_memory(pkg, cuda):
+    """Systems of one block post nothing: the first solve of 2,000 of them
+    takes their tables (250 bytes a system), not posts (278 KB each)."""
+    import torch
+    s = pkg.meshgen.pressure_system((5, 4, 3), seed=60)
+    B = pkg.krylov.DeviceBatch([s.matrix] * 2000)
+    x = torch.zeros(B.rows, dtype=torch.float64, device=cuda)
+    r = torch.from_numpy(np.tile(s.b, 2000)).to(cuda)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    res = B.solve("cg", 1, x, r, np.full(2000, 8, np.int32), np.zeros(2000))
+    assert free - torch.cuda.mem_get_info()[0] < 64 << 20
+    assert np.all(res["niter"] == 9)
+    B.close()
+
+
 def test_batch_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
     mg = pkg.meshgen
     systems = [mg.pressure_system((40, 40, 41), seed=50), mg.pressure_system((41, 39, 38), seed=51)]
