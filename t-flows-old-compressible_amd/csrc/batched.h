@@ -82,6 +82,7 @@ class Batch {
         std::vector<int> index, blk_sys;   // the batch's number of each; each block's position in sys
         int grid = 0, R = 0;
         size_t lds = 0;
+        bool alone = false;                // no block waits for another
         DevArray<ResidentSystem> d_sys;
         DevArray<int> d_blk;
     };

@@ -103,7 +103,9 @@ bool launch_cgs_window(const Sell<double>& A, const ResidentArgs<double>& a, con
                        double* q, double* u2, int grid, hipStream_t s);
 // LDS of system s in a launch of R rows per thread (the most of any system)
 size_t batch_window_lds(const ResidentSystem& s, int R);
-bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, uint32_t tag,
-                            hipStream_t s);
+// (alone: every system is one block, so that no block waits and the grid
+// need not be on the device at once)
+bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, bool alone,
+                            uint32_t tag, hipStream_t s);
 
 }  // namespace tflows

@@ -49,7 +49,8 @@
 // device-scope accesses, not bandwidth, bounds it.
 //
 // Every wait ends: the grid is at most one block per CU (the host checks
-// that the device holds it at once), and a wait longer than wait_ticks
+// that the device holds it at once; a batch of one-block systems has no wait
+// and may have more), and a wait longer than wait_ticks
 // (another process held the CUs) raises the fault word, on which every
 // block stops; the host then restores the vectors and runs the
 // kernel-per-phase form.
@@ -1085,9 +1086,9 @@ void launch_resident_deps(int n, int rows, int grid, const int* rowptr, const in
     hipLaunchKernelGGL(k_resident_deps, dim3(grid), dim3(kBlock), 0, s, n, rows, rowptr, col, deps);
 }
 
-// Launches `kernel` on `grid` blocks if the device holds them all at once.
+// Launches `kernel` on `grid` blocks if the device holds `at_once` of them.
 template <class K, class... Args>
-static bool launch_resident(K kernel, int grid, size_t lds, hipStream_t s, const Args&... args) {
+static bool launch_resident_of(int at_once, K kernel, int grid, size_t lds, hipStream_t s, const Args&... args) {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -1096,9 +1097,13 @@ static bool launch_resident(K kernel, int grid, size_t lds, hipStream_t s, const
         (void)hipGetLastError();
         return false;
     }
-    if (per_cu <= 0 || grid > per_cu * cus) return false;
+    if (per_cu <= 0 || at_once > per_cu * cus) return false;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kResThreads), lds, s, args...);
     return true;
+}
+template <class K, class... Args>
+static bool launch_resident(K kernel, int grid, size_t lds, hipStream_t s, const Args&... args) {
+    return launch_resident_of(grid, kernel, grid, lds, s, args...);
 }
 
 template <typename Op, typename T>
@@ -1146,14 +1151,14 @@ bool launch_cgs_window(const Sell<double>& A, const ResidentArgs<double>& a, con
 }
 
 template <int N>
-static bool launch_batch(std::integral_constant<int, N>, int R, int grid, size_t lds, const ResidentSystem* sys,
-                         const int* blk_sys, uint32_t tag, hipStream_t s) {
+static bool launch_batch(std::integral_constant<int, N>, int R, int grid, size_t lds, bool alone,
+                         const ResidentSystem* sys, const int* blk_sys, uint32_t tag, hipStream_t s) {
     if constexpr (N > resident_rows_per_thread<double>(false)) {
         return false;
     } else {
-        if (R <= N) return launch_resident(k_cg_window_batch<N>, grid, lds, s, sys, blk_sys, tag);
-        return launch_batch(std::integral_constant<int, window_kernel_rows(N + 1)>{}, R, grid, lds, sys, blk_sys, tag,
-                            s);
+        if (R <= N) return launch_resident_of(alone ? 1 : grid, k_cg_window_batch<N>, grid, lds, s, sys, blk_sys, tag);
+        return launch_batch(std::integral_constant<int, window_kernel_rows(N + 1)>{}, R, grid, lds, alone, sys, blk_sys,
+                            tag, s);
     }
 }
 size_t batch_window_lds(const ResidentSystem& s, int R) {
@@ -1161,9 +1166,9 @@ size_t batch_window_lds(const ResidentSystem& s, int R) {
     return sizeof(double) * (2 * (size_t)s.w.lo + (size_t)s.w.nfar * s.a.rows +
                              (size_t)K * kResThreads * (window_d_in_lds<double>(K) ? 2 : 1));
 }
-bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, uint32_t tag,
-                            hipStream_t s) {
-    return launch_batch(std::integral_constant<int, 2>{}, R, grid, lds, sys, blk_sys, tag, s);
+bool launch_cg_window_batch(const ResidentSystem* sys, const int* blk_sys, int grid, int R, size_t lds, bool alone,
+                            uint32_t tag, hipStream_t s) {
+    return launch_batch(std::integral_constant<int, 2>{}, R, grid, lds, alone, sys, blk_sys, tag, s);
 }
 
 template bool launch_cg_window<Sell<double>, double>(const Sell<double>&, const ResidentArgs<double>&,

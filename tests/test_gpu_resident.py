@@ -471,6 +471,33 @@ def test_batch_of_several_launches(pkg, cuda):
         assert _rel(a[1][q], ref[1][q]) <= 1e-12
 
 
+@pytest.mark.parametrize("larger", [0, 1])
+def test_batch_of_more_small_systems_than_blocks(pkg, cuda, larger):
+    """More one-block systems than the chip holds blocks, of two rows to the
+    most of a block: one launch, each stopping by itself; systems of several
+    blocks beside them have launches of their own."""
+    mg = pkg.meshgen
+    rng = np.random.default_rng(8)
+    shapes = [tuple(int(v) for v in rng.integers(2, 9, 3)) for _ in range(297)] + [(16, 16, 16), (2, 1, 1), (64, 8, 1)]
+    shapes += [(40, 40, 41), (19, 16, 17)] * larger
+    systems = [mg.pressure_system(sh, seed=100 + q) for q, sh in enumerate(shapes)]
+    caps = np.full(len(shapes), 500, np.int32)
+    caps[::7] = 3
+    caps[300:] = 12
+    tols = np.array([s.tol for s in systems])
+    got = _batch(pkg, cuda, systems, 0, caps, tols)
+    ref = _batch(pkg, cuda, systems, 1, caps, tols)[0]
+    for a in got:
+        assert np.array_equal(a[0]["niter"], got[0][0]["niter"])
+        for q, s in enumerate(systems):
+            assert np.array_equal(a[1][q], got[0][1][q]) and np.array_equal(a[2][q], got[0][2][q])
+            assert abs(int(a[0]["niter"][q]) - int(ref[0]["niter"][q])) <= 1, q
+            if a[0]["niter"][q] <= caps[q]:
+                assert np.linalg.norm(s.b - s.matrix.to_scipy() @ a[1][q]) < 10 * tols[q]
+            else:                      # capped after three or twelve iterations
+                assert _rel(a[1][q], ref[1][q]) <= 1e-12
+
+
 def test_batch_of_small_systems_keeps_its_memory(pkg, cuda):
     """Systems of one block post nothing: the first solve of 2,000 of them
     takes their tables (250 bytes a system), not posts (278 KB each)."""
