@@ -74,7 +74,7 @@ class Batch {
     bool persistent_ok() const { return persistent_ok_; }
 
    private:
-    std::unique_ptr<CuShare> waiting_share(int method, int prec) const;
+    std::unique_ptr<CuShare> dic_share(int prec) const;
     // CG of every system on the chip (cg_resident.hip): launches of as many
     // systems as it holds at once, one after another.
     struct ResidentWave {

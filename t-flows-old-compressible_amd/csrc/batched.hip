@@ -549,6 +549,7 @@ BatchConfig Batch::tune(int bits, int method, int prec, const Op& Aop, const Csr
                 prepare();
                 TF_CHECK(hipMemcpyAsync(st, init.data(), sizeof(SolverState) * k_, hipMemcpyHostToDevice, bs_));
                 start_solve<T, Op>(c, method, prec, Aop, A, w, S, st, hm, L, bs_, d_ready, zero_x);
+                const CuShare share(-1);
                 TF_CHECK(hipEventRecord(ev_[2], bs_));
                 launch_batch_cg_chunk<Op, T>(c, Aop, A.n, probe, w.x, w.r1, w.p, w.q, (const T*)w.D, S, st, hm,
                                              bar_.p, k_, pfault_.p, wait_ticks_, bs_);
@@ -716,6 +717,7 @@ void Batch::run(int bits, int method, int prec, const Op& Aop, const Csr<T>& A, 
     int slot = 0;
     long long issued = 0, launched = 0;
     bool all_done = false;
+    std::unique_ptr<CuShare> share(form == kFormPersistent ? new CuShare(-1) : nullptr);
     while (issued < limit) {
         TF_CHECK(hipGraphLaunch(exec, bs_));
         issued += C;
@@ -759,6 +761,7 @@ void Batch::run(int bits, int method, int prec, const Op& Aop, const Csr<T>& A, 
         slot = other;
     }
     TF_CHECK(hipStreamSynchronize(bs_));
+    share.reset();
     if (form == kFormPersistent) {
         int fault = 0;
         TF_CHECK(hipMemcpy(&fault, pfault_.p, sizeof(int), hipMemcpyDeviceToHost));
@@ -953,7 +956,9 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
     }
     bool ok = true;
     out.resize(k_);
+    int at_once = 0;                     // blocks of a launch that wait for each other
     for (auto& wv : waves_) {
+        if (!wv->alone) at_once = std::max(at_once, wv->grid);
         int post = 0;
         for (size_t j = 0; j < wv->sys.size(); ++j) {
             ResidentSystem& s = wv->sys[j];
@@ -977,6 +982,7 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
         TF_CHECK(hipMemcpyAsync(wv->d_blk.p, wv->blk_sys.data(), sizeof(int) * wv->blk_sys.size(),
                                 hipMemcpyHostToDevice, bs_));
     }
+    const std::unique_ptr<CuShare> share(at_once ? new CuShare(at_once) : nullptr);
     for (;;) {
         for (auto& wv : waves_) {
             ok = ok && launch_cg_window_batch(wv->d_sys.p, wv->d_blk.p, wv->grid, wv->R, wv->lds, wv->alone, res_tag_,
@@ -1001,18 +1007,17 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
     return false;
 }
 
-// The device's CUs, where the launches of a solve may wait for each other's
-// blocks (DIC sweeps, the persistent form).
-std::unique_ptr<CuShare> Batch::waiting_share(int method, int prec) const {
-    const bool waits = prec == 2 ? sys_->dic_form() >= 2 : method == 0;
-    return std::unique_ptr<CuShare>(waits ? new CuShare(-1) : nullptr);
+// The device's CUs for a DIC solve, whose sweeps' wavefronts wait for each
+// other throughout.
+std::unique_ptr<CuShare> Batch::dic_share(int prec) const {
+    return std::unique_ptr<CuShare>(prec == 2 && sys_->dic_form() >= 2 ? new CuShare(-1) : nullptr);
 }
 
 void Batch::solve(int method, int prec, double* x, double* r1, const int* cap, const double* tol,
                   SolveResult* res, hipStream_t s) {
     check_method(method, prec);
     method = kernel_method(method);
-    const std::unique_ptr<CuShare> share = waiting_share(method, prec);
+    const std::unique_ptr<CuShare> share = dic_share(prec);
     join(s);
     const KrylovVectors<double> w = vectors64();
     std::vector<SolverState> init(k_);
@@ -1077,7 +1082,7 @@ void Batch::solve_mixed(int method, int prec, double* x, const double* b, double
                         hipStream_t s) {
     check_method(method, prec);
     method = kernel_method(method);
-    const std::unique_ptr<CuShare> share = waiting_share(method, prec);
+    const std::unique_ptr<CuShare> share = dic_share(prec);
     if (!(inner_rtol > 0.0 && inner_rtol < 1.0)) throw std::invalid_argument("inner_rtol must be in (0, 1)");
     join(s);
     const int n = n_tot_, T = tile0_[k_];

@@ -360,6 +360,45 @@ def test_two_threads(pkg, cuda):
             assert g[0] == alone[q][0] and np.array_equal(g[1], alone[q][1]) and np.array_equal(g[2], alone[q][2])
 
 
+def test_kernel_form_batch_leaves_the_chip_to_others(pkg, cuda):
+    """A batch whose kernels do not wait for each other (form 1) does not hold
+    the CUs: an on-chip solve of another thread ends while the batch, 100 times
+    as long, still runs, and both give what they give alone."""
+    import time
+    import torch
+    mg = pkg.meshgen
+    systems = [mg.pressure_system((40, 40, 41), seed=90 + q) for q in range(4)]
+    caps, tols = np.full(4, 6000, np.int32), np.zeros(4)
+    single = mg.pressure_system((32, 32, 32), seed=95)
+    want = _solve(pkg, cuda, single, 1, 60, 0.0)
+    B = pkg.krylov.DeviceBatch([s.matrix for s in systems])
+    B.set_form(1)
+    x = torch.zeros(B.rows, dtype=torch.float64, device=cuda)
+    b = torch.from_numpy(np.concatenate([s.b for s in systems])).to(cuda)
+    ends, xs = {}, []
+
+    def batch():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            xx, rr = x.clone(), b.clone()
+            torch.cuda.current_stream().synchronize()
+            B.solve("cg", 1, xx, rr, caps, tols)
+            ends["batch"] = time.perf_counter()
+            xs.append(xx.cpu().numpy())
+
+    batch()                            # tuned, and the graph captured
+    t = threading.Thread(target=batch)
+    t.start()
+    time.sleep(0.01)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got = _solve(pkg, cuda, single, 1, 60, 0.0)
+    ends["single"] = time.perf_counter()
+    t.join()
+    assert ends["single"] < ends["batch"]
+    assert got[0] == want[0] and np.array_equal(got[1], want[1])
+    assert np.array_equal(xs[0], xs[1], equal_nan=True)
+    B.close()
+
+
 @pytest.mark.parametrize("shape", ["one_slice_short", "last_block_short", "blocks_64", "two_step_ragged", "rows_16"])
 def test_mixed_matches(pkg, cuda, monkeypatch, shape):
     """The FP32 iterations of the reliable-update solve: both forms reach the
