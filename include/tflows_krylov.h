@@ -293,7 +293,7 @@ int tflows_batch_layout(tflows_batch b, int32_t* rows, int64_t* entries, int32_t
  * of finished systems are handed to running ones (rebalance != 0). */
 int tflows_batch_configure(tflows_batch b, int32_t grid, int32_t lanes, int32_t chunk, int32_t rebalance);
 /* Configuration in use for (bits = 64 or 32, method, prec) and the number
- * of rebalances so far. */
+ * of rebalances so far.  Form 3 has no launch shape to fix: 0, 0, 0. */
 int tflows_batch_config(tflows_batch b, int32_t bits, int32_t method, int32_t prec, int32_t* grid, int32_t* lanes,
                         int32_t* chunk, int32_t* rebalances);
 /* Launch form of the iterations.  1: one launch per kernel of an
@@ -305,12 +305,17 @@ int tflows_batch_config(tflows_batch b, int32_t bits, int32_t method, int32_t pr
  * the device holds at once.  Form 2 exists for CG and BiCG (which runs
  * through the CG kernels) with prec 0 or 1, in FP64 and for the FP32
  * inner solves; other solves run form 1.  Both forms give the same bits.
- * 0 (the default) lets the autotuner time both on the caller's systems
- * and keep the faster.  A persistent launch whose barrier wait exceeds
+ * 0 (the default): FP64 CG and BiCG with prec 0 or 1 run on the chip where
+ * every system is a natural-order box or as regular (rows of at most 7
+ * entries on at most 7 column offsets) and no launch shape or grouping is
+ * fixed, in form 3: each system has its own blocks, which keep its vectors
+ * and rows for up to 1024 iterations a launch.  Elsewhere the autotuner times
+ * forms 1 and 2 on the caller's systems and keeps the faster.  A persistent launch whose barrier wait exceeds
  * TFLOWS_BARRIER_WAIT_MS (default 2000 ms; other work holding the CUs) is
  * abandoned and the solve runs again in form 1, which the batch keeps. */
 int tflows_batch_set_form(tflows_batch b, int32_t form);
-/* The form (1 or 2) in use for (bits, method, prec); -1 on error. */
+/* The form in use for (bits, method, prec): 1 or 2, or 3 once a solve has run
+ * on the chip (set_form takes 0, 1 and 2); -1 on error. */
 int32_t tflows_batch_form(tflows_batch b, int32_t bits, int32_t method, int32_t prec);
 /* How the systems share the iterations (form 1, prec 0 or 1).  1: every
  * system from the first iteration.  2: consecutive systems packed into
@@ -320,8 +325,8 @@ int32_t tflows_batch_form(tflows_batch b, int32_t bits, int32_t method, int32_t 
  * both on the caller's systems and keeps the faster.  Bits may differ
  * between the two, as between grids.  No counterpart in the reference. */
 int tflows_batch_set_groups(tflows_batch b, int32_t mode);
-/* The number of groups the solves of (bits, method, prec) run in (1: all
- * at once); -1 on error. */
+/* The number of groups, or form 3's launches, the solves of (bits, method,
+ * prec) run in (1: all at once); -1 on error. */
 int32_t tflows_batch_groups(tflows_batch b, int32_t bits, int32_t method, int32_t prec);
 /* FP64 solve of all K systems with `method` / `prec` (as tflows_solve):
  * x, r1 device arrays (r1 in: b, out: final residual); cap[k], tol[k] per

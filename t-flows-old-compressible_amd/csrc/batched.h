@@ -21,10 +21,11 @@ struct BatchConfig {
     int grid = 0;    // blocks per launch (multiple of 8)
     int lanes = 0;   // SpMV form: lanes per row (1, 2, 4, 8)
     int chunk = 0;   // iterations per graph replay
-    int form = 0;    // 1: one launch per kernel; 2: one persistent launch per chunk (CG, Jacobi / none)
+    int form = 0;    // 1: one launch per kernel; 2: one persistent launch per chunk (CG, Jacobi / none);
+                     // 3 (reported only): on the chip
     int groups = 0;  // 1: every system from the start; 2: in groups that fit the MALL, one after another
 };
-enum { kFormKernels = 1, kFormPersistent = 2 };
+enum { kFormKernels = 1, kFormPersistent = 2, kFormChip = 3 };
 
 class Batch {
    public:
@@ -54,10 +55,12 @@ class Batch {
                      const double* tol, double inner_rtol, int max_outer, SolveResult* res, int* outer_steps,
                      hipStream_t s);
 
-    // Fixed launch configuration (0 = let the autotuner choose), and the
-    // configuration in use for (precision bits, method, prec).
+    // Fixed launch configuration (0 = let the autotuner choose), the kernel
+    // forms' configuration for (precision bits, method, prec), and the one in
+    // use: that, or the on-chip form, which has no launch shape to fix.
     void configure(const BatchConfig& c) { fixed_ = c; }
     BatchConfig config_for(int bits, int method, int prec) const;
+    BatchConfig config_in_use(int bits, int method, int prec) const;
     void set_rebalance(bool on) { rebalance_ = on; }
     int rebalances() const { return rebalances_; }
     // 0: the autotuner picks the form; 1 / 2 fix it (2 applies where the
@@ -67,7 +70,8 @@ class Batch {
     // 2: systems in groups whose working sets fit the 256 MB MALL, one group
     // after another (form 1, Jacobi or no preconditioner)
     void set_groups(int mode) { groups_ = mode; }
-    // the number of groups the solves of (bits, method, prec) run in
+    // the number of groups (on the chip: launches) the solves of (bits,
+    // method, prec) run in
     int groups_in_use(int bits, int method, int prec) const;
     // false once a persistent launch gave up waiting on its barriers; the
     // batch then keeps the per-kernel form
@@ -86,6 +90,7 @@ class Batch {
         DevArray<ResidentSystem> d_sys;
         DevArray<int> d_blk;
     };
+    bool on_chip(int method, int prec) const;   // no form, launch shape or grouping is fixed
     bool resident_waves();               // builds waves_; false: this batch's rows or sizes do not allow it
     bool run_resident(int prec, const KrylovVectors<double>& w, const std::vector<SolverState>& init,
                       const std::function<void()>& prepare, std::vector<SolverState>& out);

@@ -417,7 +417,20 @@ BatchConfig Batch::config_for(int bits, int method, int prec) const {
     return c;
 }
 
+bool Batch::on_chip(int method, int prec) const {
+    const bool chosen = form_ || groups_ || fixed_.grid || fixed_.lanes || fixed_.chunk;
+    return method == 0 && prec != 2 && !chosen && resident_ != 0 && cg_resident_enabled();
+}
+
+BatchConfig Batch::config_in_use(int bits, int method, int prec) const {
+    if (bits != 64 || resident_ != 1 || !on_chip(method, prec)) return config_for(bits, method, prec);
+    BatchConfig c;
+    c.form = kFormChip;
+    return c;
+}
+
 int Batch::groups_in_use(int bits, int method, int prec) const {
+    if (config_in_use(bits, method, prec).form == kFormChip) return (int)waves_.size();
     return config_for(bits, method, prec).groups == 2 ? (int)mall_groups(bits, method).size() : 1;
 }
 
@@ -1034,9 +1047,7 @@ void Batch::solve(int method, int prec, double* x, double* r1, const int* cap, c
     const Csr<double> A = sys_->csr();
     std::vector<SolverState> out;
     // on the chip, unless a form, launch shape or grouping is fixed
-    const bool chosen = form_ || groups_ || fixed_.grid || fixed_.lanes || fixed_.chunk;
-    if (method != 0 || prec == 2 || chosen || !cg_resident_enabled() || !resident_waves() ||
-        !run_resident(prec, w, init, prepare, out))
+    if (!on_chip(method, prec) || !resident_waves() || !run_resident(prec, w, init, prepare, out))
         sys_->with_op64(bs_, [&](const auto& Aop) {
             run<double, std::decay_t<decltype(Aop)>>(64, method, prec, Aop, A, w, partials_.p, st_.p, hm_, init, false,
                                                      false, prepare, out);

@@ -452,14 +452,14 @@ int32_t tflows_batch_groups(tflows_batch b, int32_t bits, int32_t method, int32_
 
 int32_t tflows_batch_form(tflows_batch b, int32_t bits, int32_t method, int32_t prec) {
     int32_t v = -1;
-    if (guarded([&] { v = b->batch->config_for(bits, tflows::kernel_method(method), prec).form; })) return -1;
+    if (guarded([&] { v = b->batch->config_in_use(bits, tflows::kernel_method(method), prec).form; })) return -1;
     return v;
 }
 
 int tflows_batch_config(tflows_batch b, int32_t bits, int32_t method, int32_t prec, int32_t* grid, int32_t* lanes,
                         int32_t* chunk, int32_t* rebalances) {
     return guarded([&] {
-        const tflows::BatchConfig c = b->batch->config_for(bits, tflows::kernel_method(method), prec);
+        const tflows::BatchConfig c = b->batch->config_in_use(bits, tflows::kernel_method(method), prec);
         if (grid) *grid = c.grid;
         if (lanes) *lanes = c.lanes;
         if (chunk) *chunk = c.chunk;

@@ -529,8 +529,9 @@ class DeviceBatch:
         _check(self.lib.tflows_batch_configure(self.handle, grid, lanes, chunk, 1 if rebalance else 0))
 
     def set_form(self, form: int):
-        """0: tuned; 1: one launch per kernel; 2: one persistent launch per
-        chunk of iterations (CG / BiCG with prec 0 or 1)."""
+        """0: on the chip where CG / BiCG with prec 0 or 1 fits it, else
+        tuned; 1: one launch per kernel; 2: one persistent launch per chunk of
+        iterations (CG / BiCG with prec 0 or 1)."""
         _check(self.lib.tflows_batch_set_form(self.handle, form))
 
     def set_groups(self, mode: int):
@@ -539,6 +540,8 @@ class DeviceBatch:
         _check(self.lib.tflows_batch_set_groups(self.handle, mode))
 
     def config(self, method: str = "cg", prec: int = 1, bits: int = 64) -> dict:
+        """The launch configuration in use; form 3 (after a solve on the
+        chip) has no grid, lanes or chunk to fix and reports 0."""
         g, l, c, r = (C.c_int32(0) for _ in range(4))
         _check(self.lib.tflows_batch_config(self.handle, bits, METHODS[method], prec, C.byref(g), C.byref(l),
                                             C.byref(c), C.byref(r)))

@@ -466,6 +466,9 @@ def _batch(pkg, cuda, systems, form, caps, tols, prec=1, b=None):
         res = B.solve("cg", prec, xx, rr, caps, tols, fin_in=np.full(len(systems), 0.5))
         torch.cuda.synchronize()
         out.append((res, [v.cpu().numpy() for v in B.split(xx)], [v.cpu().numpy() for v in B.split(rr)]))
+    out.append(B.config("cg", prec))
+    B.configure(*(out[-1][k] for k in ("grid", "lanes", "chunk")))    # what it reports may be set again
+    assert B.config("cg", prec) == out[-1]
     B.close()
     return out
 
@@ -484,7 +487,10 @@ def test_batch_matches_kernel_form(pkg, cuda, prec):
     b = [s.b.copy() for s in systems]
     b[4][:] = 0.0                      # ||b|| < tol: the early exit
     got = _batch(pkg, cuda, systems, 0, caps, tols, prec, b)
-    ref = _batch(pkg, cuda, systems, 1, caps, tols, prec, b)[0]
+    ref = _batch(pkg, cuda, systems, 1, caps, tols, prec, b)
+    assert got.pop() == dict(grid=0, lanes=0, chunk=0, rebalances=0, form=3, groups=1)
+    assert ref.pop()["form"] == 1
+    ref = ref[0]
     for a in got:
         assert np.array_equal(a[0]["niter"], got[0][0]["niter"])
         for q, s in enumerate(systems):
@@ -526,6 +532,8 @@ def test_batch_of_more_small_systems_than_blocks(pkg, cuda, larger):
     tols = np.array([s.tol for s in systems])
     got = _batch(pkg, cuda, systems, 0, caps, tols)
     ref = _batch(pkg, cuda, systems, 1, caps, tols)[0]
+    cfg = got.pop()
+    assert cfg["form"] == 3 and cfg["groups"] == 1 + larger      # launches
     for a in got:
         assert np.array_equal(a[0]["niter"], got[0][0]["niter"])
         for q, s in enumerate(systems):
@@ -559,7 +567,7 @@ def test_batch_wait_bound_falls_back(pkg, cuda, monkeypatch, capfd):
     caps, tols = np.full(2, 30, np.int32), np.zeros(2)
     whole = _batch(pkg, cuda, systems, 0, caps, tols)[0]
     monkeypatch.setenv("TFLOWS_BARRIER_WAIT_MS", "0")
-    got = _batch(pkg, cuda, systems, 0, caps, tols)[0]
-    assert capfd.readouterr().err.count("gave up waiting") == 1
+    got, _, cfg = _batch(pkg, cuda, systems, 0, caps, tols)
+    assert capfd.readouterr().err.count("gave up waiting") == 1 and cfg["form"] in (1, 2)
     for q in range(2):
         assert got[0]["niter"][q] == 31 and _rel(got[1][q], whole[1][q]) <= 1e-11
