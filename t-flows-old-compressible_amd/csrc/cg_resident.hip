@@ -547,6 +547,7 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             const int l = k * kResThreads + tid;
+            if (l >= nloc) continue;                     // alfa may be infinite
             xv[k] = xv[k] + alfa * lp[l];                // CG.f90:227
             rv[k] = rv[k] - alfa * zq[k];                // CG.f90:228
         }
@@ -774,7 +775,9 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
         for (int k = 0; k < R; ++k) {
             const int l = k * kResThreads + t;
             if (l < nloc) xv[k] = xv[k] + alfa * own[l];            // CG.f90:227
-            rv[k] = rv[k] - alfa * zq[k];                           // CG.f90:228
+            // an infinite alfa must not turn FinRes into NaN past the rows
+            // (a replacement's norm is FinRes in the mixed solve)
+            if (MIXED || l < nloc) rv[k] = rv[k] - alfa * zq[k];    // CG.f90:228
         }
         ++it;
         if (MIXED && it - it0 == a.chunk) break;
@@ -954,7 +957,9 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
                     xv[k] = xv[k] + alfa * p;                       // :286-288
                     return p;
                 },
-                [&](int k, T y) { rv[k] = rv[k] - alfa * y; }))     // :315-317
+                [&](int k, T y) {
+                    if (k * kResThreads + t < nloc) rv[k] = rv[k] - alfa * y;      // :315-317; alfa may be infinite
+                }))
             return;
         ++it;
     }

@@ -115,6 +115,27 @@ def test_shared_offsets_beyond_the_window(pkg, oracle, cuda, monkeypatch):
         assert _rel(out["1"][1], out["0"][1]) <= 1e-12 and _residuals_agree(s, out["1"], out["0"])
 
 
+@pytest.mark.parametrize("n", [2, 514, 9000])
+@pytest.mark.parametrize("op", ["sliced", "csr"])
+def test_breakdown_reports_what_the_kernels_do(pkg, cuda, monkeypatch, n, op):
+    """(p, A p) = 0 exactly: alfa, x and FinRes become infinite; the threads
+    past the last row must not turn the norm into NaN."""
+    import scipy.sparse as sp
+    A = sp.csr_matrix((np.ones(2 * n), (np.repeat(np.arange(n), 2), (np.arange(n)[:, None] // 2 * 2 + [0, 1]).ravel())),
+                      shape=(n, n))
+    A.data[:] = np.tile([0.0, 1.0, -1.0, 0.0], n // 2)
+    s = pkg.meshgen.LinearSystem(pkg.meshgen.from_scipy(A), np.ones(n), np.zeros(n), 0.0, 0, 1, {})
+    if op == "csr":
+        monkeypatch.setenv("TFLOWS_FP64_OP", "csr")
+    out = {}
+    for mode in ("1", "0"):
+        monkeypatch.setenv("TFLOWS_CG_RESIDENT", mode)
+        out[mode] = _solve(pkg, cuda, s, 0, 1, 0.0)
+    a, b = out["1"], out["0"]
+    assert a[0] == b[0] and a[0][2] == np.inf
+    assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2]) and np.isinf(a[1]).all()
+
+
 def _graph(pkg, n, offsets, rows=None, seed=3):
     """Symmetric diagonally dominant matrix: entries i, i + d for the offsets,
     and for a few rows i, i + 2, i + 5, ... (`rows`: how many more)."""
