@@ -12,12 +12,15 @@ namespace {
 
 constexpr int kLanes = 64;             // lanes of a wavefront: the posts it polls at once
 constexpr int kXcds = 8;
-// one block up to this many rows: its synchronisations are block barriers
+// One block up to this many rows: its synchronisations are block barriers
+// (CG, us an iteration, one block / several of 1024 rows: 1,331 rows 3.1 / 4.8,
+// 2,744 3.9 / 5.2, 4,096 4.7 / 5.2).
 constexpr int kResOneBlockRows = 4096;
-// else blocks of at least this many: below it the synchronisation of more
-// blocks costs more than the shorter row sums save; up to twice as many
-// where that keeps to the blocks that synchronise in one step (84,480 rows,
-// locality order: 64 blocks 11.6 ms, 80 blocks 13.9)
+// Else blocks of at least this many (2048: 5.0 -> 5.7 at 4,913 rows, 9.0 -> 9.9
+// at 175,616; 512: 5.0 -> 5.1 and 9.0 -> 8.2), up to twice as many where that
+// keeps to the 64 blocks that synchronise in one step (64 / more blocks: 85,184
+// rows 7.4 / 8.6, 97,336 7.4 / 7.9, 125,000 7.6 / 9.1, locality order 7.5 / 8.7;
+// at 216,000 rows in 64 blocks 9.0 -> 10.4).
 constexpr int kResMinRows = 1024;
 
 }  // namespace

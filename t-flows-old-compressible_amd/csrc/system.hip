@@ -1277,9 +1277,11 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
     KrylovVectors<double> w = vectors(x, r1);
     // CG and CGS on the chip where they fit (they read no workspace that they
     // or their set-up have not written).  CGS of a system of one block keeps
-    // the kernels: on small pressure matrices its count follows the reference
-    // loop's within one only with their summation by 256-row tiles (12^3: 134
-    // iterations, 128 on the chip, from rounding alone)
+    // the kernels: on small pressure matrices, a hundred iterations, its count
+    // follows the reference loop's within one only with their summation by
+    // 256-row tiles (12^3: 134 iterations, 128 on the chip, from rounding
+    // alone); on larger ones neither form's does, and on velocity matrices
+    // both do
     ResidentShape shape;
     if (method == 0 && prec != 2) shape = resident_cg_shape();
     if (method == 2 && prec != 2 && !res_off_ && cg_resident_enabled()) shape = resident_shape(n_, kCgsRows);

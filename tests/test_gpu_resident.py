@@ -241,6 +241,20 @@ def test_cgs_matches(pkg, oracle, cuda, monkeypatch, case, prec):
         assert ac[0][0] <= 600 and ac[0][2] < s.tol and true[0] < 10 * max(s.tol, true[1])
 
 
+@pytest.mark.parametrize("shape", [(17, 17, 17), (25, 24, 23), (31, 30, 29)])
+@pytest.mark.parametrize("renumber", [False, True])
+def test_cgs_count_of_momentum_matrices(pkg, oracle, cuda, shape, renumber):
+    """The velocity matrices CGS is run on converge in a few dozen iterations,
+    in which rounding shifts the last one by one at most: the on-chip count is
+    the reference loop's.  (On pressure matrices of these sizes, hundreds of
+    iterations, either form's count is up to 6 % from it, by rounding.)"""
+    for seed in (1, 2, 3):
+        s = pkg.meshgen.momentum_system(shape, seed=seed, renumber=renumber)
+        res = _solve(pkg, cuda, s, 1, 2000, s.tol, "cgs")[0]
+        ref = oracle.run("cgs", s.matrix, s.b, prec=1, niter=2000, tol=s.tol)
+        assert abs(res[0] - ref["niter"]) <= 1 and res[2] < s.tol
+
+
 @pytest.mark.parametrize("boxes", [[(16, 16, 16)] * 8, [(40, 40, 41)] * 2, [(70, 60, 25)] * 3, [(40, 40, 41)]])
 def test_cgs_of_boxes_numbered_one_after_another(pkg, cuda, monkeypatch, boxes):
     """A block's halo is loaded whole: rows of a zone's last plane lack the
