@@ -19,10 +19,11 @@
 // so an iteration costs two synchronisations, one write of z, one read of
 // the halo's z, and gathers from LDS.
 //
-// k_cg_stream: any matrix (rows of any length, columns anywhere): the rows
-// are read every iteration and p is published, which takes a third
-// synchronisation (A: a block waits for the blocks its columns reach).  It
-// sums over the same rows in the same order, so both give the same bits.
+// k_cg_stream: rows that k_cg_window does not hold (more than 7 entries, or
+// columns beyond the halo): they are read every iteration and p is
+// published, which takes a third synchronisation (A: a block waits for the
+// blocks its columns reach).  It sums over the same rows in the same order,
+// so both give the same bits.
 //
 // Process/CG.f90:113-259 per iteration, every value formed with the
 // reference's operations in the reference's order (each row's products added
@@ -44,8 +45,9 @@
 // 491,111 26.1 -> 9.1, 979,902 35.8 -> 12.6; locality order 230,580 rows
 // 18.2 -> 8.5, 506,880 28.9 -> 10.4; k_cg_stream (CSR rows) 65,600 rows
 // 14.8 -> 11.7, 491,111 28.5 -> 20.7, 979,902 40.8 -> 34.3.  At 491,111 rows
-// (256 blocks, 2.1 GHz) an iteration is 7400 cycles of synchronisation C,
-// 6100 of B, 3400 of halo, 1200 of row sums and 3000 of the rest: latency of
+// (256 blocks, 2.35 GHz) an iteration is 20,900 cycles: 5900 to 7400 of
+// synchronisation C, 6100 of B, 3200 to 4400 of halo, 1100 of row sums, 1100
+// of waiting for the published z and 2100 of the rest: latency of
 // device-scope accesses, not bandwidth, bounds it.
 //
 // Every wait ends: the grid is at most one block per CU (the host checks
@@ -184,7 +186,7 @@ __device__ __forceinline__ double poll_sum(const uint64_t* slots, int k, int str
 // whole block agrees).  Up to a wavefront of blocks each reads all posts;
 // above that the first block of each eighth adds its eighth's posts and posts
 // the sum, and every block reads eight: all blocks reading all posts took
-// 9000 cycles at 256 blocks, two steps take 6200 (one at 32 blocks: 3300).
+// 10,000 cycles at 256 blocks, two steps take 6000 (one at 32 blocks: 3500).
 template <int NV>
 __device__ __forceinline__ bool resident_sum(int tid, double (&v)[NV], uint64_t* slots, int nblk, int blk, uint32_t tag,
                                              const Waiter& wt, int* s_fail, double* sm) {
@@ -623,8 +625,9 @@ __device__ __forceinline__ void halo_update(int t, const CoherentVec<T>& zin, T*
 // MIXED: the FP32 iterations of a residual-replacement solve.  A thread's
 // rows are summed in FP32, the threads' and blocks' sums in FP64: the mean
 // error of x against 64 bits over 26 solves of 0.26 to 2.1 M rows is 2.9e-7,
-// with every sum in FP32 3.8e-7 (one launch per kernel: 4.0e-7).  The second
-// word of a post takes 128^3 from 7.07 to 7.19 ms.
+// with every sum in FP32 3.8e-7 (one launch per kernel: 4.0e-7), and with the
+// threads' sums in FP64 but FP32 posts 3.3e-7.  450 iterations of 128^3 take
+// 7.19, 7.07 and 7.15 ms.
 template <typename Op, bool SHARED, int R, bool MIXED, typename T>
 __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, const int G,
                                           const int blk) {
