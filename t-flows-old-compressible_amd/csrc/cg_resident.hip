@@ -93,7 +93,9 @@ __device__ __forceinline__ void coherent_store(float* p, float v) {
 // block reads them in kPostCopies copies, one for the blocks of each XCD
 // (one copy: 7500 cycles against 3700 at 32 blocks).  Each word carries 32
 // bits of the value and the tag.
-constexpr int kValueWords = 2;         // words of a value
+template <typename P> struct PostWords;
+template <> struct PostWords<double> { static constexpr int n = 2; };
+template <> struct PostWords<float> { static constexpr int n = 1; };
 
 __device__ __forceinline__ void post_word(uint64_t* w, uint32_t v, uint32_t tag) {
     __hip_atomic_store(w, ((uint64_t)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -103,12 +105,20 @@ __device__ __forceinline__ void post_value(uint64_t* w, int stride, double v, ui
     post_word(w, (uint32_t)b, tag);
     post_word(w + stride, (uint32_t)(b >> 32), tag);
 }
+__device__ __forceinline__ void post_value(uint64_t* w, int, float v, uint32_t tag) {
+    post_word(w, __builtin_bit_cast(uint32_t, v), tag);
+}
 // true (and v) when every word of the value carries the tag
 __device__ __forceinline__ bool read_value(const uint64_t* w, int stride, uint32_t tag, double& v) {
     const uint64_t a = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint64_t b = __hip_atomic_load(w + stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     v = __builtin_bit_cast(double, (a & 0xffffffffu) | (b << 32));
     return (uint32_t)(a >> 32) == tag && (uint32_t)(b >> 32) == tag;
+}
+__device__ __forceinline__ bool read_value(const uint64_t* w, int, uint32_t tag, float& v) {
+    const uint64_t a = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = __builtin_bit_cast(float, (uint32_t)a);
+    return (uint32_t)(a >> 32) == tag;
 }
 
 // Waits of one launch: bounded by the wall clock and the fault word.
@@ -133,15 +143,15 @@ struct Waiter {
 // Sum over the block of value k of every thread, in wavefront k's lanes.  The
 // values go through LDS and one wavefront adds them: a cross-lane sum in
 // every wavefront cost 4 x 40 instructions on each SIMD.
-template <int NV>
-__device__ __forceinline__ double block_partial(int tid, const double (&v)[NV], double* sm) {
+template <typename T, int NV>
+__device__ __forceinline__ T block_partial(int tid, const T (&v)[NV], T* sm) {
     const int lane = tid & (kWave - 1), w = tid / kWave;
 #pragma unroll
     for (int k = 0; k < NV; ++k) sm[k * kResThreads + tid] = v[k];
     __syncthreads();
-    double s = 0.0;
+    T s = T(0);
     if (w < NV) {
-        double t[kResWaves];
+        T t[kResWaves];
 #pragma unroll
         for (int i = 0; i < kResWaves; ++i) t[i] = sm[w * kResThreads + i * kWave + lane];
         s = t[0];
@@ -156,20 +166,21 @@ __device__ __forceinline__ double block_partial(int tid, const double (&v)[NV], 
 template <int NV>
 __device__ __forceinline__ void block_total(double (&v)[NV], double* sm) {
     __shared__ double tot[NV];
-    const double s = block_partial<NV>(threadIdx.x, v, sm);
+    const double s = block_partial<double, NV>(threadIdx.x, v, sm);
     if (threadIdx.x % kWave == 0 && threadIdx.x / kWave < NV) tot[threadIdx.x / kWave] = s;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = tot[k];
 }
 
-// Polls block b's post of value k where `use`, and returns the sum over the
-// wavefront's lanes in every one of them.
+// Polls block b's post of value k where `use`, and returns the FP64 sum over
+// the wavefront's lanes in every one of them.
+template <typename P>
 __device__ __forceinline__ double poll_sum(const uint64_t* slots, int k, int stride, int b, bool use, uint32_t tag,
                                            const Waiter& wt, int* s_fail) {
-    double got = 0.0;
+    P got = P(0);
     if (use) {
-        const uint64_t* s = slots + k * kValueWords * stride + b;
+        const uint64_t* s = slots + k * PostWords<P>::n * stride + b;
         unsigned polls = 0;
         uint64_t t0 = 0;
         while (!read_value(s, stride, tag, got))
@@ -178,41 +189,47 @@ __device__ __forceinline__ double poll_sum(const uint64_t* slots, int k, int str
                 break;
             }
     }
-    return wave_sum(got);
+    return wave_sum((double)got);
 }
 
 // Sums of NV values over the block, then over the `nblk` blocks (posted in
-// `slots`).  Valid in every thread; false when the wait was given up (the
-// whole block agrees).  Up to a wavefront of blocks each reads all posts;
-// above that the first block of each eighth adds its eighth's posts and posts
-// the sum, and every block reads eight: all blocks reading all posts took
-// 10,000 cycles at 256 blocks, two steps take 6000 (one at 32 blocks: 3500).
-template <int NV>
-__device__ __forceinline__ bool resident_sum(int tid, double (&v)[NV], uint64_t* slots, int nblk, int blk, uint32_t tag,
-                                             const Waiter& wt, int* s_fail, double* sm) {
+// `slots`), these in FP64.  Valid in every thread; false when the wait was
+// given up (the whole block agrees).  Up to a wavefront of blocks each reads
+// all posts; above that the first block of each eighth adds its eighth's posts
+// and posts the sum, and every block reads eight: all blocks reading all posts
+// took 10,000 cycles at 256 blocks, two steps take 6000 (one at 32 blocks:
+// 3500).
+template <typename T, int NV>
+__device__ __forceinline__ bool resident_sum(int tid, const T (&v)[NV], double (&sum)[NV], uint64_t* slots, int nblk,
+                                             int blk, uint32_t tag, const Waiter& wt, int* s_fail, T* sm) {
     __shared__ double tot[NV];
+    constexpr int kWords = PostWords<T>::n, kWords2 = PostWords<double>::n;
     const int lane = tid & (kWave - 1), w = tid / kWave;
-    double s = block_partial<NV>(tid, v, sm);
+    const T mine = block_partial<T, NV>(tid, v, sm);
+    double s = mine;
     if (w < NV && nblk > 1) {
-        const bool flat = nblk <= kWave;
-        const int m = nblk / kNumXcd, g = flat ? 0 : blk / m;        // above kWave blocks, a multiple of 8
-        bool poster = true;
-        if (!flat) {
-            if (lane == 0) post_value(slots + w * kValueWords * kPostStride + blk, kPostStride, s, tag);
-            poster = blk == g * m;
-            if (poster) s = poll_sum(slots, w, kPostStride, blk + lane, lane < m, tag, wt, s_fail);
-            slots += kPostCopies * kPostSite;
+        if (nblk <= kWave) {
+            if (lane < kPostCopies)
+                post_value(slots + lane * kPostSite + w * kWords * kPostStride + blk, kPostStride, mine, tag);
+            s = poll_sum<T>(slots + (blockIdx.x & (kPostCopies - 1)) * kPostSite, w, kPostStride, lane, lane < nblk, tag,
+                            wt, s_fail);
+        } else {
+            const int m = nblk / kNumXcd, g = blk / m;       // above kWave blocks, a multiple of 8
+            if (lane == 0) post_value(slots + w * kWords * kPostStride + blk, kPostStride, mine, tag);
+            uint64_t* const second = slots + kPostCopies * kPostSite;
+            if (blk == g * m) {
+                s = poll_sum<T>(slots, w, kPostStride, blk + lane, lane < m, tag, wt, s_fail);
+                if (lane < kPostCopies)
+                    post_value(second + lane * kPostSecond + w * kWords2 * kNumXcd + g, kNumXcd, s, tag);
+            }
+            s = poll_sum<double>(second + (blockIdx.x & (kPostCopies - 1)) * kPostSecond, w, kNumXcd, lane,
+                                 lane < kNumXcd, tag, wt, s_fail);
         }
-        const int stride = flat ? kPostStride : kNumXcd, copy = flat ? kPostSite : kPostSecond;
-        if (poster && lane < kPostCopies)
-            post_value(slots + lane * copy + w * kValueWords * stride + (flat ? blk : g), stride, s, tag);
-        s = poll_sum(slots + (blockIdx.x & (kPostCopies - 1)) * copy, w, stride, lane, lane < (flat ? nblk : kNumXcd),
-                     tag, wt, s_fail);
     }
     if (w < NV && lane == 0) tot[w] = s;
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = tot[k];
+    for (int k = 0; k < NV; ++k) sum[k] = tot[k];
     return *s_fail == 0;
 }
 
@@ -458,7 +475,7 @@ template <typename Op, int R, typename T = typename OpValue<Op>::type>
 __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T> a) {
     extern __shared__ __align__(16) char res_lds[];
     T* lp = reinterpret_cast<T*>(res_lds);           // p of this block's rows
-    __shared__ double sm[2 * kResThreads];
+    __shared__ T sm[2 * kResThreads];
     __shared__ int s_fail, s_done;
     SolverState* st = a.st;
     const int tid = threadIdx.x;
@@ -508,8 +525,9 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
             v[0] += rv[k] * rv[k];                       // ||r||^2, CG.f90:250
             v[1] += rv[k] * zq[k];                       // rho, CG.f90:174
         }
-        if (!resident_sum<2>(tid, v, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
-        err = sqrt((double)v[0]);
+        double sum[2];
+        if (!resident_sum(tid, v, sum, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
+        err = sqrt(sum[0]);
         if (err < tol) {                                 // CG.f90:93-108, :248-255
             stop = true;
             niter = it;
@@ -521,7 +539,7 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
             break;
         }
         if (it - it0 == a.chunk) break;
-        const T rho = v[1];
+        const T rho = (T)sum[1];
         const bool first = it == 0;
         const T beta = first ? T(0) : rho / rho_old;     // CG.f90:183
         rho_old = rho;
@@ -544,8 +562,9 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
             zq[k] = l < nloc ? stream_row(A, rb + l, g) : T(0);     // CG.f90:193-199
             pq[0] += lp[l] * zq[k];                                 // CG.f90:216
         }
-        if (!resident_sum<1>(tid, pq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
-        const T alfa = rho / pq[0];                      // CG.f90:219
+        double spq[1];
+        if (!resident_sum(tid, pq, spq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
+        const T alfa = rho / (T)spq[0];                      // CG.f90:219
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             const int l = k * kResThreads + tid;
@@ -622,17 +641,16 @@ __device__ __forceinline__ void halo_update(int t, const CoherentVec<T>& zin, T*
 // far regions of w; else the halo is the window of columns the block reaches
 // (deps).  LDS: halo below, own rows, halo above, far regions.
 //
-// MIXED: the FP32 iterations of a residual-replacement solve.  A thread's
-// rows are summed in FP32, the threads' and blocks' sums in FP64: the mean
-// error of x against 64 bits over 26 solves of 0.26 to 2.1 M rows is 2.9e-7,
-// with every sum in FP32 3.8e-7 (one launch per kernel: 4.0e-7), and with the
-// threads' sums in FP64 but FP32 posts 3.3e-7.  450 iterations of 128^3 take
-// 7.19, 7.07 and 7.15 ms.
+// MIXED: the FP32 iterations of a residual-replacement solve.  A block's sum
+// is FP32, the sums over blocks FP64: the mean error of x against 64 bits over
+// 26 solves of 0.26 to 2.1 M rows is 3.1e-7, with every sum in FP32 3.8e-7 (one
+// launch per kernel 4.0e-7), with the threads' sums in FP64, too, 2.9e-7.  450
+// iterations of 128^3 take 7.07, 7.02 and 7.19 ms.
 template <typename Op, bool SHARED, int R, bool MIXED, typename T>
 __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, const int G,
                                           const int blk) {
     extern __shared__ __align__(16) char res_lds[];
-    __shared__ double sm[2 * kResThreads];
+    __shared__ T sm[2 * kResThreads];
     __shared__ int s_fail, s_done;
     SolverState* st = a.st;
     const int tid = threadIdx.x;
@@ -699,9 +717,10 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
         for (int q = 0; q < w.nfar; ++q) first_p(far_run<T>(w, rb, a.rows, q));
     double err64 = 0.0;
     if (MIXED) {                    // the FP64 norm of the replacement before this launch (site E)
+        __shared__ double sm64[kResThreads];
         double e[1] = {0.0};
         for (int b = tid; b < a.nE; b += kResThreads) e[0] += a.partE[b];
-        block_total<1>(e, sm);
+        block_total<1>(e, sm64);
         err64 = sqrt(e[0]);
     }
     uint32_t tag = a.tag;
@@ -723,8 +742,8 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
             if (G > 1 && l < nloc) coherent_store(a.z + rb + l, zq[k]);
         }
         __builtin_amdgcn_s_waitcnt(0);               // this wave's z has reached memory before the block posts
-        double sum[2] = {v[0], v[1]};
-        if (!resident_sum<2>(t, sum, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
+        double sum[2];
+        if (!resident_sum(t, v, sum, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
         err = sqrt(sum[0]);
         if (MIXED && it == it0) {                    // after a replacement the FP64 norm decides
             err = err_rep = err64;
@@ -771,8 +790,8 @@ __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a,
             if (l < nloc) pq[0] += own[l] * zq[k];                  // CG.f90:216
             if (R > 2) asm volatile("" : "+v"(zq[k]));              // one row's gathers in registers at a time
         }
-        double spq[1] = {pq[0]};
-        if (!resident_sum<1>(t, spq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
+        double spq[1];
+        if (!resident_sum(t, pq, spq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
         const T alfa = rho / (T)spq[0];                             // CG.f90:219
 #pragma unroll
         for (int k = 0; k < R; ++k) {
@@ -833,7 +852,7 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
                                                             const T* __restrict__ shadow, T* __restrict__ qg,
                                                             T* __restrict__ u2g) {
     extern __shared__ __align__(16) char res_lds[];
-    __shared__ double sm[2 * kResThreads];
+    __shared__ T sm[2 * kResThreads];
     __shared__ int s_fail, s_done;
     SolverState* st = a.st;
     const int tid = threadIdx.x;
@@ -922,8 +941,9 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
             v[0] += rv[k] * rv[k];
             v[1] += rv[k] * sv[k];                                  // rho, CGS.f90:118-122
         }
-        if (!resident_sum<2>(t, v, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
-        err = sqrt((double)v[0]);
+        double sum[2];
+        if (!resident_sum(t, v, sum, a.slotC, G, blk, ++tag, wt, &s_fail, sm)) return;
+        err = sqrt(sum[0]);
         if (err < tol) {
             stop = true;
             niter = it;
@@ -935,7 +955,7 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
             break;
         }
         if (it - it0 == a.chunk) break;
-        const T rho = v[1];
+        const T rho = (T)sum[1];
         const bool first = it == 0;
         const T beta = first ? T(0) : rho / rho_old;
         rho_old = rho;
@@ -951,8 +971,9 @@ __global__ __launch_bounds__(kResThreads) void k_cgs_window(Op A, ResidentArgs<T
                          rs[0] += sv[k] * y;                        // (r2, v)  :215-219
                      }))
             return;
-        if (!resident_sum<1>(t, rs, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
-        const T alfa = rho / rs[0];                                 // :220
+        double srs[1];
+        if (!resident_sum(t, rs, srs, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
+        const T alfa = rho / (T)srs[0];                                 // :220
         if (!product(
                 [&](int k) {
                     qv[k] = u1[k] - alfa * qv[k];                   // :226-228

@@ -466,8 +466,8 @@ def test_mixed_matches(pkg, cuda, monkeypatch, shape):
 
 def test_mixed_error_against_64_bits(pkg, cuda, monkeypatch):
     """Capped mixed solves against FP64 CG of the same cap.  Both forms round
-    the same FP32 vectors and the on-chip one sums them in FP64, so its mean
-    error is no larger; single solves scatter (a factor of 1.8 either way, so
+    the same FP32 vectors and the on-chip one adds its blocks' sums in FP64, so
+    its mean error is no larger; single solves scatter (a factor of 1.8 either way, so
     the mean of 16 by about 15 %, and 1.25 is the ratio's bar)."""
     import torch
     mg = pkg.meshgen
