@@ -250,7 +250,9 @@ class System {
     // the CSR arrays themselves (the same row sums bit for bit).
     // TFLOWS_FP64_OP=csr / =sliced fixes the form; otherwise the first use
     // times both and keeps the faster.
-    Sell<double> sell64(hipStream_t s);
+    // (unless_done: new values are not filled in when this solve is already
+    // over on the device; the caller then marks them stale)
+    Sell<double> sell64(hipStream_t s, const SolverState* unless_done = nullptr);
     template <class F>
     void with_op64(hipStream_t s, F&& f) {
         if (op64_sliced(s)) f(sell64(s));

@@ -215,12 +215,14 @@ template bool pairs_symmetric<float>(const DevArray<int>&, int64_t, const float*
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_slot_values(int64_t count, const int* __restrict__ map,
-                                                        const T* __restrict__ src, T* __restrict__ dst) {
+                                                        const T* __restrict__ src, T* __restrict__ dst,
+                                                        const SolverState* unless_done) {
+    if (unless_done && unless_done->done) return;
     const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (e < count) dst[e] = map[e] < 0 ? T(0) : src[map[e]];
 }
 
-Sell<double> System::sell64(hipStream_t s) {
+Sell<double> System::sell64(hipStream_t s, const SolverState* unless_done) {
     if (!sell64_built_) {
         std::vector<int> rp(n_ + 1), cl(nnz_), off, col, map;
         TF_CHECK(hipMemcpyAsync(rp.data(), rowptr_.p, sizeof(int) * (n_ + 1), hipMemcpyDeviceToHost, s));
@@ -291,11 +293,11 @@ Sell<double> System::sell64(hipStream_t s) {
             // values that differ from their mirrors: the full form from now on
             sym64_refused_ = true;
             sell64_built_ = false;
-            return sell64(s);
+            return sell64(s, unless_done);
         }
         hipLaunchKernelGGL((k_slot_values<double>), dim3((unsigned)((sell64_entries_ + kBlock - 1) / kBlock)),
                            dim3(kBlock), 0, s, sell64_entries_, (const int*)sell64_map_.p, (const double*)val_.p,
-                           sell64_val_.p);
+                           sell64_val_.p, unless_done);
         TF_CHECK(hipGetLastError());
         sell64_valid_ = true;
     }
@@ -1318,11 +1320,18 @@ SolveResult System::solve_impl(int method, int prec, double* x, double* r1, int 
         if (method == 0) launch_cgf_check(false, sites(), (const double*)nullptr, state_.p, mirror_, s);   // CG.f90:93-108
         else launch_check(ctx(), 1, sites(), state_.p, mirror_, s);
         auto launch = [&](const ResidentArgs<double>& a) {
-            if (method == 2) return launch_cgs_window(sell64(s), a, win64_, w.r2, w.q, w.u2, shape.grid, s);
-            return window ? launch_cg_window(sell64(s), a, win64_, shape.grid, s)
+            if (method == 2) return launch_cgs_window(sell64(s, state_.p), a, win64_, w.r2, w.q, w.u2, shape.grid, s);
+            return window ? launch_cg_window(sell64(s, state_.p), a, win64_, shape.grid, s)
                           : launch_cg_stream(A, a, shape.grid, s);
         };
+        // a solve that was over before its first iteration has not filled in
+        // new values
+        struct Stale {
+            bool &valid, filled;
+            ~Stale() { valid = valid && filled; }
+        } stale{sell64_valid_, sell64_valid_};
         resident = run_resident(shape, sp, launch, w, state_.p, h, h2, s);
+        stale.filled = stale.filled || (resident && h2.it > 0);
         if (!resident && method == 0)
             launch_cgf_init_z(n_, (const double*)w.r1, (const double*)w.D, w.u1, sites(), state_.p, s);
     }

@@ -136,6 +136,38 @@ def test_breakdown_reports_what_the_kernels_do(pkg, cuda, monkeypatch, n, op):
     assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2]) and np.isinf(a[1]).all()
 
 
+@pytest.mark.parametrize("method", ["cg", "cgs"])
+@pytest.mark.parametrize("renumber", [False, True])
+def test_new_values_after_a_solve_that_ends_at_once(pkg, cuda, method, renumber):
+    """A solve that is over before its first iteration (b = 0) does not fill
+    new values into the operator; the next one does."""
+    import torch
+    s = pkg.meshgen.momentum_system((25, 24, 23), seed=9, renumber=renumber)
+    n, b = s.matrix.n, torch.from_numpy(s.b.copy()).to(cuda)
+    values = torch.from_numpy(s.matrix.aval.copy()).to(cuda)
+
+    def run(ds, rhs, cap=8):
+        x, r = torch.zeros(n, dtype=torch.float64, device=cuda), rhs.clone()
+        res = ds.solve(method, 1, x, r, cap, 0.0 if cap else 1e-9)
+        return res, x.cpu().numpy(), r.cpu().numpy()
+
+    ds = pkg.krylov.DeviceSystem(s.matrix)
+    run(ds, b)
+    want = {}
+    for scale in (3.0, 0.25):
+        ds.set_values(values * scale)
+        want[scale] = run(ds, b)
+    for scale in (3.0, 0.25):
+        ds.set_values(values * scale)
+        x, r = torch.zeros(n, dtype=torch.float64, device=cuda), torch.zeros(n, dtype=torch.float64, device=cuda)
+        assert ds.solve(method, 1, x, r, 8, 1e-9)[0] == 0 and not x.any()
+        assert run(ds, b, 0)[0][0] == 1             # a cap of 0 ends before the first iteration, too
+        got = run(ds, b)
+        assert got[0] == want[scale][0] and np.array_equal(got[1], want[scale][1])
+        assert np.array_equal(got[2], want[scale][2])
+    ds.close()
+
+
 def _graph(pkg, n, offsets, rows=None, seed=3):
     """Symmetric diagonally dominant matrix: entries i, i + d for the offsets,
     and for a few rows i, i + 2, i + 5, ... (`rows`: how many more)."""
