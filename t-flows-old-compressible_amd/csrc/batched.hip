@@ -971,7 +971,6 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
     out.resize(k_);
     int at_once = 0;                     // blocks of a launch that wait for each other
     for (auto& wv : waves_) {
-        if (!wv->alone) at_once = std::max(at_once, wv->grid);
         int post = 0;
         for (size_t j = 0; j < wv->sys.size(); ++j) {
             ResidentSystem& s = wv->sys[j];
@@ -994,6 +993,7 @@ bool Batch::run_resident(int prec, const KrylovVectors<double>& w, const std::ve
                                 hipMemcpyHostToDevice, bs_));
         TF_CHECK(hipMemcpyAsync(wv->d_blk.p, wv->blk_sys.data(), sizeof(int) * wv->blk_sys.size(),
                                 hipMemcpyHostToDevice, bs_));
+        if (post) at_once = std::max(at_once, wv->grid);
     }
     const std::unique_ptr<CuShare> share(at_once ? new CuShare(at_once) : nullptr);
     for (;;) {

@@ -1097,7 +1097,11 @@ CuShare::CuShare(int blocks) : dev_(0), blocks_(blocks) {
     CuPool& p = g_cu_pools[dev_];
     std::unique_lock<std::mutex> lk(p.m);
     if (p.cap == 0) p.cap = std::max(1, device_cus());
-    if (blocks_ < 0 || blocks_ > p.cap) blocks_ = p.cap;
+    // blocks go to the XCDs in turn: as many of each XCD as the fullest one
+    // gets, so that no launch waits for a CU of one XCD that another launch
+    // holds while that waits for a CU of another XCD
+    if (blocks_ >= 0) blocks_ = std::min(p.cap, (blocks_ + kNumXcd - 1) / kNumXcd * kNumXcd);
+    else blocks_ = p.cap;
     const uint64_t mine = p.next++;
     p.cv.wait(lk, [&] { return p.serving == mine && p.used + blocks_ <= p.cap; });
     p.used += blocks_;

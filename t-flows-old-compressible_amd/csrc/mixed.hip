@@ -647,7 +647,7 @@ SolveResult System::solve_mixed_reliable_impl(int prec, double* x, const double*
     const DiffSell32 A32 = resident ? sell32(s) : DiffSell32{};
     std::unique_ptr<CuShare> share;
     if (resident) {
-        share.reset(new CuShare(shape.grid));
+        if (shape.grid > 1) share.reset(new CuShare(shape.grid));
         TF_CHECK(hipMemcpyAsync(sp.keep, x, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     }
     ResidentArgs<float> ra{};

@@ -1192,7 +1192,7 @@ bool System::run_resident(const ResidentShape& shape, const ResidentSpace& sp,
                           const std::function<bool(const ResidentArgs<double>&)>& launch,
                           const KrylovVectors<double>& w, SolverState* st, const SolverState& h0, SolverState& h,
                           hipStream_t s) {
-    const CuShare share(shape.grid);
+    const std::unique_ptr<CuShare> share(shape.grid > 1 ? new CuShare(shape.grid) : nullptr);
     if (!sp.deps_ready && shape.grid > 1)
         launch_resident_deps(n_, shape.rows, shape.grid, rowptr_.p, col_.p, sp.deps, s);
     ResidentArgs<double> a{};

@@ -427,6 +427,49 @@ def test_two_threads(pkg, cuda):
             assert g[0] == alone[q][0] and np.array_equal(g[1], alone[q][1]) and np.array_equal(g[2], alone[q][2])
 
 
+def test_batch_beside_small_systems(pkg, cuda, capfd):
+    """An on-chip batch whose launch has about as many blocks as the chip, no
+    multiple of the XCDs', beside solves of five blocks from another thread:
+    neither waits for CUs that the other holds, and both give what they give
+    alone."""
+    import torch
+    mg = pkg.meshgen
+    shapes = [(61, 60, 59), (61, 59, 47), (53, 51, 49)] + [(17, 241, 1)] * 9
+    systems = [mg.pressure_system(s, seed=110 + q) for q, s in enumerate(shapes)]
+    k = len(systems)
+    B = pkg.krylov.DeviceBatch([s.matrix for s in systems])
+    b = torch.from_numpy(np.concatenate([s.b for s in systems])).to(cuda)
+    small = mg.pressure_system((17, 17, 17), seed=96)
+    want = _solve(pkg, cuda, small, 1, 40, 0.0)
+    runs = {"batch": [], "small": []}
+
+    def batch():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(8):
+                x, r = torch.zeros_like(b), b.clone()
+                torch.cuda.current_stream().synchronize()
+                B.solve("cg", 1, x, r, np.full(k, 60, np.int32), np.zeros(k))
+                runs["batch"].append(x.cpu().numpy())
+
+    def singles():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(30):
+                runs["small"].append(_solve(pkg, cuda, small, 1, 40, 0.0))
+
+    batch()
+    assert B.config("cg", 1)["form"] == 3
+    ts = [threading.Thread(target=f) for f in (batch, singles)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    B.close()
+    assert "gave up" not in capfd.readouterr().err
+    assert len(runs["batch"]) == 16 and len(runs["small"]) == 30
+    assert all(np.array_equal(x, runs["batch"][0]) for x in runs["batch"])
+    assert all(g[0] == want[0] and np.array_equal(g[1], want[1]) for g in runs["small"])
+
+
 def test_kernel_form_batch_leaves_the_chip_to_others(pkg, cuda):
     """A batch whose kernels do not wait for each other (form 1) does not hold
     the CUs: an on-chip solve of another thread ends while the batch, 100 times

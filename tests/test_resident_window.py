@@ -19,7 +19,7 @@ CSRC = os.path.join(REPO, "t-flows-old-compressible_amd", "csrc")
 
 
 @pytest.fixture(scope="module")
-def checker():
+def program():
     cxx = shutil.which("g++")
     if cxx is None:
         pytest.skip("no host C++ compiler")
@@ -31,8 +31,8 @@ def checker():
     return out
 
 
-def test_halo_rows_are_waited_for(checker):
-    r = subprocess.run([checker], capture_output=True, text=True, timeout=120)
+def test_halo_rows_are_waited_for(program):
+    r = subprocess.run([program], capture_output=True, text=True, timeout=120)
     print(r.stdout)
     assert r.returncode == 0 and "ALL OK" in r.stdout, r.stdout + r.stderr
     beyond = {l.split()[1]: int(l.split("beyond=")[1].split()[0]) for l in r.stdout.splitlines() if "beyond=" in l}
