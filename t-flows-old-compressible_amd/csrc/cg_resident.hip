@@ -564,7 +564,7 @@ __global__ __launch_bounds__(kResThreads) void k_cg_stream(Op A, ResidentArgs<T>
         }
         double spq[1];
         if (!resident_sum(tid, pq, spq, a.slotB, G, blk, ++tag, wt, &s_fail, sm)) return;
-        const T alfa = rho / (T)spq[0];                      // CG.f90:219
+        const T alfa = rho / (T)spq[0];                  // CG.f90:219
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             const int l = k * kResThreads + tid;
