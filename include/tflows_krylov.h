@@ -123,7 +123,7 @@ int tflows_solve(tflows_system s, int32_t method, int32_t prec, double* x, doubl
 /* tflows_solve without any allocation: the solver state, the reduction
  * partials and the work vectors (D, p, q, z, and x / r1 in the internal
  * order of a renumbered system) live in one fixed device array of the
- * library (each GPU holds its own copy, about 48 MiB, until the process
+ * library (each GPU holds its own copy, about 49 MiB, until the process
  * ends), so
  * the call makes no hipMalloc / hipFree / hipHostMalloc and no allocating
  * library call.  No counterpart in the reference: it is for callers that
