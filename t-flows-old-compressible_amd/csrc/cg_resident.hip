@@ -173,9 +173,17 @@ __device__ __forceinline__ void block_total(double (&v)[NV], double* sm) {
     for (int k = 0; k < NV; ++k) v[k] = tot[k];
 }
 
+// wave_sum of values in the first eight lanes, 0 in the others: the same bits
+__device__ __forceinline__ double octet_sum(double v) {
+    v += dpp_d<kQuadSwap1>(v);
+    v += dpp_d<kQuadSwap2>(v);
+    v += dpp_d<kRowHalfMirror>(v);
+    return readlane_d(v, 0);
+}
+
 // Polls block b's post of value k where `use`, and returns the FP64 sum over
-// the wavefront's lanes in every one of them.
-template <typename P>
+// the wavefront's lanes (OCTET: the first eight) in every one of them.
+template <typename P, bool OCTET = false>
 __device__ __forceinline__ double poll_sum(const uint64_t* slots, int k, int stride, int b, bool use, uint32_t tag,
                                            const Waiter& wt, int* s_fail) {
     P got = P(0);
@@ -189,21 +197,21 @@ __device__ __forceinline__ double poll_sum(const uint64_t* slots, int k, int str
                 break;
             }
     }
-    return wave_sum((double)got);
+    return OCTET ? octet_sum((double)got) : wave_sum((double)got);
 }
 
-// Sums of NV values over the block, then over the `nblk` blocks (posted in
-// `slots`), these in FP64.  Valid in every thread; false when the wait was
-// given up (the whole block agrees).  Up to a wavefront of blocks each reads
-// all posts; above that the first block of each eighth adds its eighth's posts
-// and posts the sum, and every block reads eight: all blocks reading all posts
-// took 10,000 cycles at 256 blocks, two steps take 6000 (one at 32 blocks:
-// 3500).
+// Sums of NV values over the block, then over the `nblk` blocks: posted in
+// `slots` in the values' type, added in FP64.  Valid in every thread; false
+// when the wait was given up (the whole block agrees).  Up to a wavefront of
+// blocks each reads all posts; above that the first block of each eighth adds
+// its eighth's posts and posts the sum, and every block reads eight: all
+// blocks reading all posts took 10,000 cycles at 256 blocks, two steps take
+// 6000 (one at 32 blocks: 3500).
 template <typename T, int NV>
 __device__ __forceinline__ bool resident_sum(int tid, const T (&v)[NV], double (&sum)[NV], uint64_t* slots, int nblk,
                                              int blk, uint32_t tag, const Waiter& wt, int* s_fail, T* sm) {
     __shared__ double tot[NV];
-    constexpr int kWords = PostWords<T>::n, kWords2 = PostWords<double>::n;
+    constexpr int kWords = PostWords<T>::n;
     const int lane = tid & (kWave - 1), w = tid / kWave;
     const T mine = block_partial<T, NV>(tid, v, sm);
     double s = mine;
@@ -220,10 +228,10 @@ __device__ __forceinline__ bool resident_sum(int tid, const T (&v)[NV], double (
             if (blk == g * m) {
                 s = poll_sum<T>(slots, w, kPostStride, blk + lane, lane < m, tag, wt, s_fail);
                 if (lane < kPostCopies)
-                    post_value(second + lane * kPostSecond + w * kWords2 * kNumXcd + g, kNumXcd, s, tag);
+                    post_value(second + lane * kPostSecond + w * kWords * kNumXcd + g, kNumXcd, (T)s, tag);
             }
-            s = poll_sum<double>(second + (blockIdx.x & (kPostCopies - 1)) * kPostSecond, w, kNumXcd, lane,
-                                 lane < kNumXcd, tag, wt, s_fail);
+            s = poll_sum<T, true>(second + (blockIdx.x & (kPostCopies - 1)) * kPostSecond, w, kNumXcd, lane,
+                                  lane < kNumXcd, tag, wt, s_fail);
         }
     }
     if (w < NV && lane == 0) tot[w] = s;
@@ -642,10 +650,11 @@ __device__ __forceinline__ void halo_update(int t, const CoherentVec<T>& zin, T*
 // (deps).  LDS: halo below, own rows, halo above, far regions.
 //
 // MIXED: the FP32 iterations of a residual-replacement solve.  A block's sum
-// is FP32, the sums over blocks FP64: the mean error of x against 64 bits over
-// 26 solves of 0.26 to 2.1 M rows is 3.1e-7, with every sum in FP32 3.8e-7 (one
-// launch per kernel 4.0e-7), with the threads' sums in FP64, too, 2.9e-7.  450
-// iterations of 128^3 take 7.07, 7.02 and 7.19 ms.
+// and the posts are FP32, the posts are added in FP64: the mean error of x
+// against 64 bits over 26 solves of 0.26 to 2.1 M rows is 3.0e-7, with every
+// sum in FP32 3.8e-7 (one launch per kernel 4.0e-7), with FP64 posts 3.1e-7,
+// with the threads' sums in FP64, too, 2.9e-7.  Against every sum in FP32 300
+// iterations take 1.0 % more at 614,125 rows (FP64 posts 3.6 %), none at 2.1 M.
 template <typename Op, bool SHARED, int R, bool MIXED, typename T>
 __device__ __forceinline__ void cg_window(const Op& A, const ResidentArgs<T>& a, const WindowShape& w, const int G,
                                           const int blk) {
